@@ -1025,7 +1025,7 @@ std::tuple<at::Tensor, at::Tensor> knn(const at::Tensor& xb, const at::Tensor& x
   const bool bf = xb.scalar_type() == at::kBFloat16;
   TORCH_CHECK(bf || xb.scalar_type() == at::kFloat, "database must be fp32 or bf16");
   TORCH_CHECK(xb.size(1) == xq.size(1), "dimension mismatch");
-  TORCH_CHECK(k >= 1 && docqa_knn_kpad(k) > 0, "k must be in [1, 64]");
+  TORCH_CHECK(k >= 1 && k <= 64, "k must be in [1, 64]");
   const int N = xb.size(0), d = xb.size(1), nq = xq.size(0);
   c10::DeviceGuard g(xb.device());
   auto out_d = at::empty({nq, k}, xq.options());
@@ -1035,14 +1035,15 @@ std::tuple<at::Tensor, at::Tensor> knn(const at::Tensor& xb, const at::Tensor& x
     out_i.fill_(-1);
     return {out_d, out_i};
   }
-  const int nblk = docqa_knn_workspace_blocks(N);
-  const int kp = docqa_knn_kpad(k);
-  auto ws_d = at::empty({nq, nblk, kp}, xq.options());
-  auto ws_i = at::empty({nq, nblk, kp}, xq.options().dtype(at::kInt));
+  auto on16 = [](const at::Tensor& t) { return (uintptr_t)t.data_ptr() % 16 ? t.clone() : t; };
+  const auto x = on16(xb), q = on16(xq);
+  int qc, rc;
+  size_t bytes;
+  docqa_knn_plan(N, nq, d, bf ? 1 : 0, (int)k, &qc, &rc, &bytes);
+  auto ws = at::empty({(int64_t)bytes}, xq.options().dtype(at::kByte));
   const float* norms = inner_product ? nullptr : xb_norms.data_ptr<float>();
-  CHECK_RC(docqa_knn(xb.data_ptr(), norms, N, d, bf ? 1 : 0, xq.data_ptr<float>(), nq, k,
-                     inner_product ? 1 : 0, ws_d.data_ptr<float>(), ws_i.data_ptr<int>(), nblk,
-                     out_d.data_ptr<float>(), out_i.data_ptr<int64_t>(), id_offset, stream()), "knn");
+  CHECK_RC(docqa_knn(x.data_ptr(), norms, N, d, bf ? 1 : 0, q.data_ptr<float>(), nq, (int)k, inner_product ? 1 : 0,
+                     ws.data_ptr(), out_d.data_ptr<float>(), out_i.data_ptr<int64_t>(), id_offset, stream()), "knn");
   return {out_d, out_i};
 }
 

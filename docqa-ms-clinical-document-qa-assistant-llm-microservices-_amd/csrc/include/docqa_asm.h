@@ -31,6 +31,13 @@ __device__ __forceinline__ void glds16(const void* gsrc, uint32_t dst_base) {
                  : "=&s"(keep) : "v"(gsrc), "s"(dst_base) : "memory");
 }
 
+// the same from a wave-uniform 64-bit base and a 32-bit byte offset per lane
+__device__ __forceinline__ void glds16_off(const void* sbase, uint32_t voff, uint32_t dst_base) {
+  unsigned keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep) : "v"(voff), "s"(sbase), "s"(dst_base) : "memory");
+}
+
 // 16-B write-through (sc1) global store: the line is not left dirty in this XCD's L2, so a
 // consumer in another workgroup of the launch needs no release fence from the producer
 // (cdna_hip_programming.md §6 Guideline 16 R1); invisible to hipcc's waitcnt pass (drain

@@ -164,11 +164,9 @@ int docqa_coarse_probes(const float* cent, const float* cnorm, int nlist, int d,
 bool docqa_pgemm_ok(int M, int N, int K);
 int docqa_pgemm(const void* A, const void* W, void* C, float* P, int M, int N, int K, int S, int epi,
                 hipStream_t s);
-int docqa_knn_workspace_blocks(int N);
-int docqa_knn_kpad(int k);
-int docqa_knn(const void* xb, const float* norms, int N, int d, int is_bf16, const float* xq,
-              int nq, int k, int metric_ip, float* ws_d, int* ws_i, int nblk, float* out_d,
-              int64_t* out_i, int64_t id_offset, hipStream_t s);
+void docqa_knn_plan(int N, int nq, int d, int is_bf16, int k, int* qc, int* rc, size_t* bytes);
+int docqa_knn(const void* xb, const float* norms, int N, int d, int is_bf16, const float* xq, int nq, int k,
+              int metric_ip, void* ws, float* out_d, int64_t* out_i, int64_t id_offset, hipStream_t s);
 
 int docqa_ivfpq_search(const float* xq, const float* centroids, const float* pq,
                        const uint8_t* codes, const int64_t* ids, const int64_t* list_off,

@@ -3,11 +3,10 @@
 // IndexFlatL2 quantizer; reference index sites semantic-indexer/indexer.py:39,41 and the
 // retriever search llm-qa/main.py:101, scaled to the 10M-vector config 2).
 //
-// The fused kNN kernel (knn.hip) keeps a register top-K per lane, which caps K at 64; the
-// operating points with recall@10 >= 0.9 at 10M vectors need nprobe 128..512.  Two kernels:
-//   1. distance tiles on MFMA, fp32 in / fp32 accumulate (v_mfma_f32_32x32x2_f32: exact
-//      fp32, the quantizer's own arithmetic): 32 queries per workgroup staged in LDS, each
-//      wave streams 32-centroid tiles; D[q, c] = ||c||^2 - 2 q.c (||q||^2 does not change a
+// The flat index's selection (knn.hip) takes K up to 64; the operating points with
+// recall@10 >= 0.9 at 10M vectors need nprobe 128..512.  Two kernels:
+//   1. distance tiles on MFMA, fp32 in / fp32 accumulate (docqa_dist.h, row-major: exact fp32,
+//      the quantizer's own arithmetic); D[q, c] = ||c||^2 - 2 q.c (||q||^2 does not change a
 //      query's probe order) -> a [nq, nlist] fp32 workspace (8 MB at nq 256, nlist 8192);
 //   2. per-query selection, one workgroup per query: MSB-first radix select over the
 //      order-preserving uint32 image of the distances (4 passes of a 256-bin LDS histogram)
@@ -15,58 +14,13 @@
 //      into LDS as (key << 32 | centroid) and bitonic-sorted, so probes come out in
 //      ascending distance, ties to the lower centroid id -- deterministic, the order of a
 //      stable CPU sort.
-#include "docqa_common.h"
-#include <float.h>
+#include "docqa_dist.h"
 
 using namespace docqa;
 
 namespace {
 
 constexpr int kMaxProbe = 512;
-
-__global__ __launch_bounds__(256) void coarse_dist_kernel(const float* __restrict__ cent,
-                                                          const float* __restrict__ cnorm, int nlist, int d,
-                                                          const float* __restrict__ xq, int nq,
-                                                          int rows_per_block, float* __restrict__ D) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int blk = blockIdx.x, q0 = blockIdx.y * 32;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int l32 = lane & 31, hh = lane >> 5;
-  float* sq = reinterpret_cast<float*>(smem);
-  for (int i = tid; i < 32 * d; i += 256) {
-    const int q = i / d, c = i - q * d;
-    sq[i] = (q0 + q < nq) ? xq[(size_t)(q0 + q) * d + c] : 0.f;
-  }
-  __syncthreads();
-  const int row_begin = blk * rows_per_block;
-  const int row_end = min(nlist, row_begin + rows_per_block);
-  const int q = q0 + l32;
-  for (int tile = row_begin + wave * 32; tile < row_end; tile += 128) {
-    const int my_row = min(tile + l32, nlist - 1);   // clamped A-operand row
-    f32x16 acc;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-    const float* a_row = cent + (size_t)my_row * d;
-    const float* b_row = sq + l32 * d;
-    for (int u = 0; u < d; u += 8) {
-      const float4 a4 = *reinterpret_cast<const float4*>(a_row + u + 4 * hh);
-      const float4 b4 = *reinterpret_cast<const float4*>(b_row + u + 4 * hh);
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a4.x, b4.x, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a4.y, b4.y, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a4.z, b4.z, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a4.w, b4.w, acc, 0, 0, 0);
-    }
-    // lane owns query l32; tile rows (r & 3) + 8 (r >> 2) + 4 hh
-    if (q < nq) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = tile + (r & 3) + 8 * (r >> 2) + 4 * hh;
-        // cnorm null: the plain product (fp32 x @ W^T -- the PQ pre-rotation)
-        if (row < row_end) D[(size_t)q * nlist + row] = cnorm ? cnorm[row] - 2.f * acc[r] : acc[r];
-      }
-    }
-  }
-}
 
 __device__ __forceinline__ unsigned order_key(float f) {
   const unsigned u = __float_as_uint(f);
@@ -161,14 +115,8 @@ __global__ __launch_bounds__(256) void coarse_select_kernel(const float* __restr
 int docqa_fp32_gemm_nt(const float* x, int nq, int d, const float* w, int n, float* out, hipStream_t s) {
   if (nq == 0) return 0;
   if (d % 8 != 0 || n <= 0 || !docqa_aligned16(x) || !docqa_aligned16(w)) return -1;
-  const size_t lds = (size_t)32 * d * 4;
-  if (lds > 160 * 1024) return -2;
-  int nblk = (n + 511) / 512;
-  if (nblk > 256) nblk = 256;
-  int rpb = (n + nblk - 1) / nblk;
-  rpb = (rpb + 127) / 128 * 128;
-  nblk = (n + rpb - 1) / rpb;
-  coarse_dist_kernel<<<dim3(nblk, (nq + 31) / 32), 256, lds, s>>>(w, nullptr, n, d, x, nq, rpb, out);
+  if ((size_t)32 * d * 4 > 160 * 1024) return -2;        // the widest rows this entry point takes
+  dist_launch<false, false>(DistArgs{w, x, nullptr, out, nullptr, n, nq, d * 4, 0, DIST_DOT}, s);
   DOCQA_CHECK_LAUNCH();
   return 0;
 }
@@ -180,15 +128,8 @@ int docqa_coarse_probes(const float* cent, const float* cnorm, int nlist, int d,
   if (nq == 0) return 0;
   if (d % 8 != 0 || nlist <= 0 || nprobe < 1 || nprobe > kMaxProbe || nprobe > nlist) return -1;
   if (!docqa_aligned16(cent) || !docqa_aligned16(xq)) return -1;
-  const size_t lds = (size_t)32 * d * 4;
-  if (lds > 160 * 1024) return -2;
-  // ~512 centroid rows per workgroup (4 tiles per wave), at most 256 row blocks
-  int nblk = (nlist + 511) / 512;
-  if (nblk > 256) nblk = 256;
-  int rpb = (nlist + nblk - 1) / nblk;
-  rpb = (rpb + 127) / 128 * 128;
-  nblk = (nlist + rpb - 1) / rpb;
-  coarse_dist_kernel<<<dim3(nblk, (nq + 31) / 32), 256, lds, s>>>(cent, cnorm, nlist, d, xq, nq, rpb, ws);
+  if ((size_t)32 * d * 4 > 160 * 1024) return -2;
+  dist_launch<false, false>(DistArgs{cent, xq, cnorm, ws, nullptr, nlist, nq, d * 4, 0, DIST_L2}, s);
   coarse_select_kernel<<<nq, 256, 0, s>>>(ws, nlist, nprobe, probes);
   DOCQA_CHECK_LAUNCH();
   return 0;

@@ -1,204 +1,239 @@
-// knn.hip -- exact brute-force k-nearest-neighbour search (FAISS IndexFlatL2 /
-// IndexFlatIP semantics) with the distance GEMM on MFMA and the top-k fused into it.
+// knn.hip -- exact brute-force k-nearest-neighbour search (FAISS IndexFlatL2 / IndexFlatIP
+// semantics): distances on MFMA (docqa_dist.h), then a selection that reads almost none of them.
 //
 // Reference parity: FAISS IndexFlatL2 search through the LangChain retriever
 // (llm-qa/main.py:101, k=3) over the 649 x 384 fp32 index written by
 // semantic-indexer/indexer.py:27,41.  FAISS returns squared L2 distances
 // ||x||^2 + ||y||^2 - 2 x.y in ascending order and int64 labels (-1 = missing).
 //
-// Kernel 1 (grid: row-blocks x query-blocks, 256 threads):
-//   * 32 queries per workgroup are staged once in LDS; the database streams from HBM.
-//   * each wave takes 32-row database tiles: X = Xb . Xq^T on MFMA
-//       fp32 database: v_mfma_f32_32x32x2_f32 (exact fp32, = FAISS fp32 semantics);
-//         lane (r, h) loads one float4 of its row = the k-slots of 4 MFMAs, the query
-//         operand uses the same dim permutation so the dot product is unchanged.
-//       bf16 database: v_mfma_f32_32x32x16_bf16 (16-B row chunks, half the HBM bytes
-//         for the 10M-vector shards).
-//   * the accumulator puts one query per lane and 16 database rows in registers, so the
-//     distance epilogue and the running per-lane top-K (register insertion network,
-//     skipped wave-wide when no lane beats its current K-th) need no data movement.
-//   * end: the 8 per-query lists (4 waves x 2 lane halves) merge through LDS into one
-//     top-K per (query, row-block) -> workspace.
-// Kernel 2 (grid nq): merges the row-block lists -> final (D, I) per query.
-#include "docqa_common.h"
-#include "docqa_topk.h"
-#include <float.h>
+// Selection.  The product kernel leaves every distance in a workspace and the least distance of
+// each 32-row tile beside it.  The K-th least of any K tile minima bounds the K-th best distance
+// from above, so a query's workgroup reads its minima (1 / 32 of the distances), bounds, and
+// fetches only the tiles whose minimum is within the bound -- about K of them.  Candidates are
+// ordered by (distance, row), so ties go to the lower row whatever order they arrive in.  Bound by
+// the product, fp32: 250,000 x 768, 256 queries, k 10 takes 809 us, and 3780 us when 32 queries at
+// a time read the rows uncoalesced and every lane kept a K-long sorted list; 2647 x 384, one
+// query, k 3 takes 17 us, 83 before (6 workgroups, ||q||^2 summed by one thread).
+//
+// Batches whose distances exceed the workspace run in pieces: queries are independent, row
+// pieces carry their K best along as (distance, row) pairs.
+#include "docqa_dist.h"
 
 using namespace docqa;
 
 namespace {
 
-template <int K, bool IP, bool BF16>
-__global__ __launch_bounds__(256) void knn_tile_kernel(
-    const void* __restrict__ xb, const float* __restrict__ xb_norms, int N, int d,
-    const float* __restrict__ xq, int nq, int rows_per_block, float* __restrict__ ws_d,
-    int* __restrict__ ws_i, int nblk) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int blk = blockIdx.x, q0 = blockIdx.y * 32;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int l32 = lane & 31, hh = lane >> 5;
+typedef unsigned long long u64;
+constexpr int kMaxK = 64;
+constexpr int kBuf = 1024;      // candidates held
+constexpr int kTiles = 1024;    // tile list
 
-  // ---- stage the 32 queries (zero padded) in LDS
-  if constexpr (BF16) {
-    uint16_t* sq = reinterpret_cast<uint16_t*>(smem);
-    for (int i = tid; i < 32 * d; i += 256) {
-      const int q = i / d, c = i - q * d;
-      sq[i] = (q0 + q < nq) ? f2bf(xq[(size_t)(q0 + q) * d + c]) : 0;
+__device__ __forceinline__ u64 cand_key(float v, uint32_t row) {
+  const uint32_t b = __float_as_uint(v);
+  return ((u64)((b & 0x80000000u) ? ~b : (b | 0x80000000u)) << 32) | row;
+}
+__device__ __forceinline__ float key_value(u64 k) {
+  const uint32_t t = (uint32_t)(k >> 32);
+  return __uint_as_float((t & 0x80000000u) ? (t & 0x7fffffffu) : ~t);
+}
+
+// buf[0, n) -> its K least in ascending order at buf[0, min(n, K)).  Few entries: every entry
+// counts those below it; many: bitonic sort.  All 256 threads call it.
+__device__ void keep_best(u64* buf, int n, int K) {
+  const int tid = threadIdx.x;
+  if (n <= 256) {
+    const u64 mine = tid < n ? buf[tid] : ~0ull;
+    int r = 0;
+    for (int j = 0; j < n; ++j) r += buf[j] < mine;      // keys are unique: rows are
+    __syncthreads();
+    if (tid < n && r < K) buf[r] = mine;
+    __syncthreads();
+    return;
+  }
+  int P = 512;
+  while (P < n) P <<= 1;
+  for (int i = n + tid; i < P; i += 256) buf[i] = ~0ull;
+  __syncthreads();
+  for (int k = 2; k <= P; k <<= 1)
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      for (int i = tid; i < P / 2; i += 256) {
+        const int a = 2 * i - (i & (j - 1)), b = a + j;
+        const u64 x = buf[a], y = buf[b];
+        if ((x > y) == ((a & k) == 0)) { buf[a] = y; buf[b] = x; }
+      }
+      __syncthreads();
     }
-  } else {
-    float* sq = reinterpret_cast<float*>(smem);
-    for (int i = tid; i < 32 * d; i += 256) {
-      const int q = i / d, c = i - q * d;
-      sq[i] = (q0 + q < nq) ? xq[(size_t)(q0 + q) * d + c] : 0.f;
-    }
+}
+
+// One query's K best of a piece of rows [row0, row0 + 32 T) and of those carried from earlier
+// pieces.  Grid: queries.
+__global__ __launch_bounds__(256) void knn_select_kernel(const float* __restrict__ D, const float* __restrict__ mins,
+                                                         int T, int ldt, int nq, int K, uint32_t row0,
+                                                         u64* __restrict__ carry, bool first, bool last,
+                                                         const float* __restrict__ xq, int d, bool ip,
+                                                         float* __restrict__ out_d, int64_t* __restrict__ out_i,
+                                                         int64_t id_offset) {
+  __shared__ u64 buf[kBuf];
+  __shared__ int list[kTiles];
+  __shared__ __attribute__((aligned(16))) float tm[256];
+  __shared__ int s_n, s_t;
+  __shared__ u64 s_bound;
+  __shared__ float s_qn[4];
+  const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const float* mq = mins + (size_t)q * ldt;
+  float mine = FLT_MAX;
+  for (int t = tid; t < T; t += 256) mine = fminf(mine, mq[t]);
+  tm[tid] = mine;
+  if (tid == 0) {
+    s_bound = cand_key(FLT_MAX, 0);                      // below it: a value that is there
+    s_t = 0;
+  }
+  if (wave == 0) {                                       // carried keys: ascending, ~0 where there are fewer
+    const u64 key = !first && lane < K ? carry[(size_t)q * K + lane] : ~0ull;
+    buf[lane] = key;
+    const u64 there = __ballot(key != ~0ull);
+    if (lane == 0) s_n = (int)__popcll(there);
+  }
+  if (last && !ip) {
+    float s = 0.f;
+    for (int c = tid; c < d; c += 256) s += xq[(size_t)q * d + c] * xq[(size_t)q * d + c];
+    s = wave_sum(s);
+    if (lane == 0) s_qn[wave] = s;
   }
   __syncthreads();
-
-  float td[K];
-  int ti[K];
-#pragma unroll
-  for (int i = 0; i < K; ++i) { td[i] = FLT_MAX; ti[i] = -1; }
-
-  const int row_begin = blk * rows_per_block;
-  const int row_end = min(N, row_begin + rows_per_block);
-  for (int tile = row_begin + wave * 32; tile < row_end; tile += 128) {
-    const int my_row = min(tile + l32, N - 1);   // clamped A-operand row
-    f32x16 acc;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-    if constexpr (BF16) {
-      const uint16_t* a_row = reinterpret_cast<const uint16_t*>(xb) + (size_t)my_row * d;
-      const uint16_t* b_row = reinterpret_cast<const uint16_t*>(smem) + l32 * d;
-      for (int s = 0; s < d; s += 16) {
-        uint4 av = *reinterpret_cast<const uint4*>(a_row + s + 8 * hh);
-        uint4 bv = *reinterpret_cast<const uint4*>(b_row + s + 8 * hh);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<bf16x8*>(&av),
-                                                      *reinterpret_cast<bf16x8*>(&bv), acc, 0, 0, 0);
+  // the bound: the K-th least of the threads' minima, each of a tile of its own
+  int r = 0;
+  for (int j = 0; j < 256; j += 4) {
+    const float4 o = *reinterpret_cast<const float4*>(tm + j);
+    r += (o.x < mine || (o.x == mine && j < tid)) + (o.y < mine || (o.y == mine && j + 1 < tid)) +
+         (o.z < mine || (o.z == mine && j + 2 < tid)) + (o.w < mine || (o.w == mine && j + 3 < tid));
+  }
+  if (r == K - 1 && mine < FLT_MAX) s_bound = cand_key(mine, 0xffffffffu);
+  __syncthreads();
+  int n = s_n;                                           // candidates held (uniform)
+  u64 bound = min(s_bound, buf[K - 1]);                  // carried rows are the lower ones: ties are theirs
+  // tiles within the bound; a list that overflows (equal rows by the thousand) is taken in parts
+  float most = key_value(bound);
+  int step = T;
+  for (int t = tid; t < T; t += 256)
+    if (mq[t] <= most && mq[t] < FLT_MAX) {
+      const int at = atomicAdd(&s_t, 1);
+      if (at < kTiles) list[at] = t;
+    }
+  __syncthreads();
+  if (s_t > kTiles) step = kTiles;
+  for (int t0 = 0; t0 < T; t0 += step) {
+    if (step != T) {
+      __syncthreads();
+      if (tid == 0) s_t = 0;
+      __syncthreads();
+      for (int t = t0 + tid; t < min(T, t0 + step); t += 256)
+        if (mq[t] <= most && mq[t] < FLT_MAX) list[atomicAdd(&s_t, 1)] = t;
+      __syncthreads();
+    }
+    const int cnt = s_t;
+    for (int i0 = 0; i0 < cnt; i0 += 8) {
+      const int i = i0 + (tid >> 5);
+      if (i < cnt) {
+        const int t = list[i];
+        const float v = D[((size_t)t * nq + q) * 32 + (tid & 31)];
+        const u64 key = cand_key(v, row0 + (uint32_t)t * 32 + (tid & 31));
+        if (v < FLT_MAX && key < bound) buf[atomicAdd(&s_n, 1)] = key;
       }
+      __syncthreads();
+      n = s_n;
+      __syncthreads();                                   // (read by all before the next group counts on)
+      if (n > kBuf - 256) {
+        keep_best(buf, n, K);
+        n = K;                                           // (n > K here)
+        bound = buf[K - 1];
+        if (tid == 0) s_n = K;
+        __syncthreads();
+      }
+    }
+    most = key_value(bound);
+  }
+  __syncthreads();
+  keep_best(buf, n, K);
+  if (tid < K) {
+    const u64 key = tid < n ? buf[tid] : ~0ull;
+    if (!last) {
+      carry[(size_t)q * K + tid] = key;
     } else {
-      const float* a_row = reinterpret_cast<const float*>(xb) + (size_t)my_row * d;
-      const float* b_row = reinterpret_cast<const float*>(smem) + l32 * d;
-      for (int u = 0; u < d; u += 8) {
-        const float4 a4 = *reinterpret_cast<const float4*>(a_row + u + 4 * hh);
-        const float4 b4 = *reinterpret_cast<const float4*>(b_row + u + 4 * hh);
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a4.x, b4.x, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a4.y, b4.y, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a4.z, b4.z, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a4.w, b4.w, acc, 0, 0, 0);
-      }
-    }
-    // epilogue: lane owns query l32; rows (r&3) + 8(r>>2) + 4hh of the tile
-    float dist[16];
-    float mn = FLT_MAX;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = tile + (r & 3) + 8 * (r >> 2) + 4 * hh;
-      float v;
-      if (row < row_end) v = IP ? -acc[r] : xb_norms[row] - 2.f * acc[r];
-      else v = FLT_MAX;
-      dist[r] = v;
-      mn = fminf(mn, v);
-    }
-    // wave-uniform skip when no lane can improve its list
-    if (__any(mn < td[K - 1])) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = tile + (r & 3) + 8 * (r >> 2) + 4 * hh;
-        if (dist[r] < td[K - 1]) topk_insert<K>(td, ti, dist[r], row);
-      }
-    }
-  }
-
-  // ---- merge the 8 lists per query through LDS (reuse the query region)
-  __syncthreads();
-  float* md = reinterpret_cast<float*>(smem);              // [32 q][8 lists][K]
-  int* mi = reinterpret_cast<int*>(smem) + 32 * 8 * K;
-  const int list = wave * 2 + hh;
-#pragma unroll
-  for (int i = 0; i < K; ++i) {
-    md[(l32 * 8 + list) * K + i] = td[i];
-    mi[(l32 * 8 + list) * K + i] = ti[i];
-  }
-  __syncthreads();
-  if (tid < 32 && q0 + tid < nq) {
-    const int q = tid;
-    int head[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) head[j] = 0;
-    const size_t ob = ((size_t)(q0 + q) * nblk + blk) * K;
-    for (int i = 0; i < K; ++i) {
-      int best = 0;
-      float bd = FLT_MAX;
-      int bi = 0x7fffffff;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        if (head[j] < K) {
-          const float v = md[(q * 8 + j) * K + head[j]];
-          const int id = mi[(q * 8 + j) * K + head[j]];
-          if (v < bd || (v == bd && id < bi)) { bd = v; bi = id; best = j; }
-        }
-      }
-      head[best]++;
-      ws_d[ob + i] = bd;
-      ws_i[ob + i] = bd == FLT_MAX ? -1 : bi;
+      const float v = key_value(key);
+      const bool ok = key != ~0ull;
+      const float qn = ip ? 0.f : (s_qn[0] + s_qn[1]) + (s_qn[2] + s_qn[3]);
+      out_d[(size_t)q * K + tid] = ok ? (ip ? -v : v + qn) : (ip ? -FLT_MAX : FLT_MAX);
+      out_i[(size_t)q * K + tid] = ok ? (int64_t)(uint32_t)key + id_offset : -1;
     }
   }
 }
 
+// bf16 database: the queries are rounded once to its type
+__global__ __launch_bounds__(256) void knn_round_kernel(const float* __restrict__ x, uint16_t* __restrict__ y, size_t n8) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n8) return;
+  float f[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) f[e] = x[i * 8 + e];
+  reinterpret_cast<uint4*>(y)[i] = pack8(f);
+}
+
+constexpr long long kPiece = 64ll << 20;     // distances a launch may leave in the workspace: 268 MB
 }  // namespace
 
-int docqa_knn_workspace_blocks(int N) {
-  int nblk = (N + 511) / 512;       // >= 512 rows (4 tiles per wave) per block
-  if (nblk > 1024) nblk = 1024;
-  return nblk < 1 ? 1 : nblk;
+// queries and rows of a piece, and the workspace in bytes (docqa_knn lays it out):
+// distances, minima, carried keys, rounded queries
+void docqa_knn_plan(int N, int nq, int d, int is_bf16, int k, int* qc, int* rc, size_t* bytes) {
+  const long long n32 = ((long long)N + 31) / 32 * 32;
+  long long c = nq, r = n32;
+  if (c * r > kPiece) {
+    c = nq < 1024 ? nq : 1024;
+    r = n32 < kPiece / c ? n32 : kPiece / c / 128 * 128;
+    c = kPiece / r < nq ? kPiece / r : nq;
+  }
+  *qc = (int)c;
+  *rc = (int)r;
+  *bytes = (size_t)c * r * 4 + (size_t)c * (r / 32) * 4 + 16 + (size_t)c * k * 8 + (is_bf16 ? (size_t)nq * d * 2 : 0);
 }
 
-template <int K, bool IP, bool BF16>
-static int launch_knn(const void* xb, const float* norms, int N, int d, const float* xq, int nq,
-                      int k, float* ws_d, int* ws_i, int nblk, float* out_d, int64_t* out_i,
-                      int64_t id_offset, hipStream_t s) {
-  int rpb = (N + nblk - 1) / nblk;
-  rpb = (rpb + 127) / 128 * 128;
-  const size_t qbytes = (size_t)32 * d * (BF16 ? 2 : 4);
-  const size_t mbytes = (size_t)32 * 8 * K * 8;
-  const size_t lds = qbytes > mbytes ? qbytes : mbytes;
-  if (lds > 160 * 1024) return -2;
-  dim3 g1(nblk, (nq + 31) / 32);
-  knn_tile_kernel<K, IP, BF16><<<g1, 256, lds, s>>>(xb, norms, N, d, xq, nq, rpb, ws_d, ws_i, nblk);
-  topk_merge_kernel<K, IP><<<nq, 256, topk_merge_lds(K), s>>>(ws_d, ws_i, nblk, xq, d, k, out_d, out_i, id_offset, nullptr);
+// xb / xq 16-byte aligned; k <= 64
+int docqa_knn(const void* xb, const float* norms, int N, int d, int is_bf16, const float* xq, int nq, int k,
+              int metric_ip, void* ws, float* out_d, int64_t* out_i, int64_t id_offset, hipStream_t s) {
+  if (nq == 0) return 0;
+  if (d % (is_bf16 ? 16 : 8) != 0 || N <= 0 || k < 1 || k > kMaxK) return -1;
+  if (!docqa_aligned16(xb) || !docqa_aligned16(xq) || !docqa_aligned16(ws)) return -1;
+  const int rowbytes = d * (is_bf16 ? 2 : 4);
+  if ((size_t)32 * rowbytes > 160 * 1024) return -2;     // the widest rows this entry point takes
+  int qc, rc;
+  size_t bytes;
+  docqa_knn_plan(N, nq, d, is_bf16, k, &qc, &rc, &bytes);
+  char* at = (char*)ws;
+  float* D = (float*)at;
+  at += (size_t)qc * rc * 4;
+  void* q16 = at;
+  if (is_bf16) {
+    at += (size_t)nq * d * 2;
+    const size_t n8 = (size_t)nq * d / 8;
+    knn_round_kernel<<<(unsigned)((n8 + 255) / 256), 256, 0, s>>>(xq, (uint16_t*)q16, n8);
+  }
+  u64* carry = (u64*)at;
+  at += (size_t)qc * k * 8;
+  float* mins = (float*)at;
+  for (int q0 = 0; q0 < nq; q0 += qc) {
+    const int c = nq - q0 < qc ? nq - q0 : qc;
+    const float* xs = xq + (size_t)q0 * d;
+    for (int r0 = 0; r0 < N; r0 += rc) {
+      const int n = N - r0 < rc ? N - r0 : rc, T = (n + 31) / 32;
+      DistArgs p{(const char*)xb + (size_t)r0 * rowbytes,
+                 is_bf16 ? (const void*)((const uint16_t*)q16 + (size_t)q0 * d) : (const void*)xs,
+                 metric_ip ? nullptr : norms + r0, D, mins, n, c, rowbytes, T, metric_ip ? DIST_IP : DIST_L2};
+      if (is_bf16) dist_launch<true, true>(p, s);
+      else dist_launch<false, true>(p, s);
+      knn_select_kernel<<<c, 256, 0, s>>>(D, mins, T, T, c, k, (uint32_t)r0, carry, r0 == 0, n == N - r0, xs, d,
+                                          metric_ip != 0, out_d + (size_t)q0 * k, out_i + (size_t)q0 * k, id_offset);
+    }
+  }
   DOCQA_CHECK_LAUNCH();
   return 0;
-}
-
-// ws_d/ws_i: [nq, nblk, Kpad] with Kpad = the template K the call selects (<= 64)
-int docqa_knn_kpad(int k) { return k <= 4 ? 4 : k <= 8 ? 8 : k <= 16 ? 16 : k <= 32 ? 32 : k <= 64 ? 64 : -1; }
-
-int docqa_knn(const void* xb, const float* norms, int N, int d, int is_bf16, const float* xq,
-              int nq, int k, int metric_ip, float* ws_d, int* ws_i, int nblk, float* out_d,
-              int64_t* out_i, int64_t id_offset, hipStream_t s) {
-  if (nq == 0) return 0;
-  if (d % (is_bf16 ? 16 : 8) != 0 || N <= 0) return -1;
-  const int kp = docqa_knn_kpad(k);
-#define KNN_CASE(KK)                                                                               \
-  case KK:                                                                                         \
-    if (metric_ip) {                                                                               \
-      return is_bf16 ? launch_knn<KK, true, true>(xb, norms, N, d, xq, nq, k, ws_d, ws_i, nblk,    \
-                                                  out_d, out_i, id_offset, s)                      \
-                     : launch_knn<KK, true, false>(xb, norms, N, d, xq, nq, k, ws_d, ws_i, nblk,   \
-                                                   out_d, out_i, id_offset, s);                    \
-    } else {                                                                                       \
-      return is_bf16 ? launch_knn<KK, false, true>(xb, norms, N, d, xq, nq, k, ws_d, ws_i, nblk,   \
-                                                   out_d, out_i, id_offset, s)                     \
-                     : launch_knn<KK, false, false>(xb, norms, N, d, xq, nq, k, ws_d, ws_i, nblk,  \
-                                                    out_d, out_i, id_offset, s);                   \
-    }
-  switch (kp) {
-    KNN_CASE(4)
-    KNN_CASE(8)
-    KNN_CASE(16)
-    KNN_CASE(32)
-    KNN_CASE(64)
-    default: return -1;
-  }
-#undef KNN_CASE
 }
