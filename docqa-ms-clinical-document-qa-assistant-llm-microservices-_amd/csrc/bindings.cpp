@@ -1062,6 +1062,16 @@ at::Tensor fp32_gemm_nt(const at::Tensor& x, const at::Tensor& w) {
   return out;
 }
 
+// fp32 [n]: squared norms of the rows of x [n, d]
+at::Tensor row_norms(const at::Tensor& x) {
+  CHECK_GPU(x); CHECK_CONTIG(x);
+  TORCH_CHECK(x.scalar_type() == at::kFloat && x.dim() == 2, "row_norms: fp32 [n, d]");
+  c10::DeviceGuard g(x.device());
+  auto out = at::empty({x.size(0)}, x.options());
+  CHECK_RC(docqa_row_norms(x.data_ptr<float>(), x.size(0), x.size(1), out.data_ptr<float>(), stream()), "row_norms");
+  return out;
+}
+
 at::Tensor coarse_probes(const at::Tensor& xq, const at::Tensor& cent, const at::Tensor& cnorm, int64_t nprobe) {
   CHECK_GPU(xq); CHECK_GPU(cent); CHECK_GPU(cnorm);
   CHECK_CONTIG(xq); CHECK_CONTIG(cent); CHECK_CONTIG(cnorm);
@@ -1290,6 +1300,7 @@ TORCH_LIBRARY(docqa, m) {
   m.def("knn(Tensor xb, Tensor xb_norms, Tensor xq, int k, bool inner_product, int id_offset) "
         "-> (Tensor, Tensor)");
   m.def("pool_l2(Tensor h, Tensor cu_seqlens, bool mean, bool normalize) -> Tensor");
+  m.def("row_norms(Tensor x) -> Tensor");
   m.def("coarse_probes(Tensor xq, Tensor cent, Tensor cnorm, int nprobe) -> Tensor");
   m.def("fp32_gemm_nt(Tensor x, Tensor w) -> Tensor");
   m.def("ivfpq_search(Tensor xq, Tensor centroids, Tensor pq, Tensor codes, Tensor ids, "
@@ -1403,6 +1414,7 @@ TORCH_LIBRARY_IMPL(docqa, CUDA, m) {
   m.impl("pgemm_partial", &pgemm_partial);
   m.impl("mgemm_argmax_val", &mgemm_argmax_val);
   m.impl("coarse_probes", &coarse_probes);
+  m.impl("row_norms", &row_norms);
   m.impl("fp32_gemm_nt", &fp32_gemm_nt);
   m.impl("dgemm_argmax_val", &dgemm_argmax_val);
   m.impl("gemv_argmax_val", &gemv_argmax_val);

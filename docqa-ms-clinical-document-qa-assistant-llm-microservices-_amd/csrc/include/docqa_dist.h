@@ -14,8 +14,8 @@
 // 64 x 64 wave tile needs 4 ds_read_b128 per 16 MFMAs of 64 clocks and is bound by the matrix
 // cores from 64 queries on (250000 x 768 by 256 queries: 778 us, 126 TFLOP/s); QT = 32 keeps one
 // query tile a wave and is bound by the database's bytes (the same by 1 query: 134 us, 5.7 TB/s).  knn_dist_small_kernel: 32 rows x 32 queries a workgroup with K split over
-// its 4 waves, operands straight from memory: the shapes whose 128-row tiles leave CUs idle
-// are bound by the latency of one K walk, which this cuts to a quarter (dist_plan).
+// its 4 or 8 waves, operands straight from memory: the shapes whose 128-row tiles leave CUs idle
+// are bound by the latency of one K walk, which this cuts (dist_plan).
 #pragma once
 #include "docqa_asm.h"
 #include "docqa_common.h"
@@ -207,16 +207,16 @@ __global__ __launch_bounds__(256, 2) void knn_dist_kernel(DistArgs p, int nqt) {
   }
 }
 
-template <bool BF16, bool TILED>
-__global__ __launch_bounds__(256, 2) void knn_dist_small_kernel(DistArgs p, int nqt) {
-  __shared__ __attribute__((aligned(16))) float part[4][32][36];    // [wave][query][row], rows padded
+template <bool BF16, bool TILED, int NW>
+__global__ __launch_bounds__(64 * NW) void knn_dist_small_kernel(DistArgs p, int nqt) {
+  __shared__ __attribute__((aligned(16))) float part[NW][32][36];    // [wave][query][row], rows padded
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hh = lane >> 5;
   const int row0 = (blockIdx.x / nqt) * 32, q0 = (blockIdx.x % nqt) * 32;
   const char* xr = (const char*)p.xb + (size_t)min(row0 + l32, p.n - 1) * p.rowbytes + hh * 16;
   const char* qr = (const char*)p.xq + (size_t)min(q0 + l32, p.nq - 1) * p.rowbytes + hh * 16;
   // this wave's 32-byte groups of K
-  const int ng = p.rowbytes >> 5, per = (ng + 3) >> 2;
+  const int ng = p.rowbytes >> 5, per = (ng + NW - 1) / NW;
   const int g0 = min(ng, wave * per), g1 = min(ng, g0 + per);
   f32x16 acc2[1][1];
   f32x16& acc = acc2[0][0];
@@ -241,10 +241,13 @@ __global__ __launch_bounds__(256, 2) void knn_dist_small_kernel(DistArgs p, int 
         make_float4(acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]);
   __syncthreads();
   // thread: 4 rows of one query; the 8 threads of a query are neighbours
+  if (tid >= 256) return;
   const int q = tid >> 3, r = (tid & 7) * 4;
-  float v[4];
+  float v[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int e = 0; e < 4; ++e) v[e] = (part[0][q][r + e] + part[1][q][r + e]) + (part[2][q][r + e] + part[3][q][r + e]);
+  for (int w = 0; w < NW; w += 2)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] += part[w][q][r + e] + part[w + 1][q][r + e];
   const float4 f = make_float4(dist_first(p, row0 + r), dist_first(p, row0 + r + 1), dist_first(p, row0 + r + 2),
                                dist_first(p, row0 + r + 3));
   float mn = dist_put<TILED>(p, row0 + r, q0 + q, f, dist_factor(p), v[0], v[1], v[2], v[3]);
@@ -277,7 +280,10 @@ inline void dist_launch(const DistArgs& p, hipStream_t s) {
   if (qt == 128) knn_dist_kernel<128, BF16, TILED><<<rt * nt(128), 256, 0, s>>>(p, nt(128));
   else if (qt == 64) knn_dist_kernel<64, BF16, TILED><<<rt * nt(64), 256, 0, s>>>(p, nt(64));
   else if (qt == 32) knn_dist_kernel<32, BF16, TILED><<<rt * nt(32), 256, 0, s>>>(p, nt(32));
-  else knn_dist_small_kernel<BF16, TILED><<<((p.n + 31) / 32) * nt(32), 256, 0, s>>>(p, nt(32));
+  // 4 waves while each has its share of a row in flight at once, else 8 (fp32, 2647 rows by 32
+  // queries, 4 / 8 waves: d 384 6.5 / 8.5 us, d 768 10.3 / 9.1)
+  else if (p.rowbytes <= 4 * 12 * 32) knn_dist_small_kernel<BF16, TILED, 4><<<((p.n + 31) / 32) * nt(32), 256, 0, s>>>(p, nt(32));
+  else knn_dist_small_kernel<BF16, TILED, 8><<<((p.n + 31) / 32) * nt(32), 512, 0, s>>>(p, nt(32));
 }
 
 }  // namespace docqa

@@ -1,6 +1,6 @@
-// docqa_topk.h -- register top-K selection and the cross-block top-K merge shared by the
-// flat kNN and IVF-PQ search kernels.  Smaller is better throughout (inner-product
-// scores are negated by the producers); ties break towards the lower candidate id.
+// docqa_topk.h -- top-K selection and the merge of partial lists that the flat and IVF-PQ search
+// kernels share.  Smaller is better throughout (inner-product scores are negated by the
+// producers); ties break towards the lower candidate id.
 #pragma once
 #include "docqa_common.h"
 #include <float.h>
@@ -125,46 +125,121 @@ __device__ void block_select_topk(const float (&td)[K], const int (&ti)[K], floa
   __syncthreads();
 }
 
-// Merge nblk partial lists per query: ws_d/ws_i [nq][nblk][K] -> out [nq][k_out].
-// Dynamic LDS: topk_merge_lds(K) bytes.
-//   qnorm_src != nullptr: add ||q||^2 (flat L2 produced ||x||^2 - 2 x.q)
-//   IP: scores were negated, flip back
-//   idmap != nullptr: translate candidate positions to stored 64-bit ids
-template <int K, bool IP>
-__global__ __launch_bounds__(256) void topk_merge_kernel(
-    const float* __restrict__ ws_d, const int* __restrict__ ws_i, int nblk,
-    const float* __restrict__ qnorm_src, int d, int k_out, float* __restrict__ out_d,
-    int64_t* __restrict__ out_i, int64_t id_offset, const int64_t* __restrict__ idmap) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char topk_smem[];
-  float* sd = reinterpret_cast<float*>(topk_smem);                 // [K] merged, ascending
-  int* si = reinterpret_cast<int*>(topk_smem + K * 4);
-  __shared__ float qn;
-  const int q = blockIdx.x, tid = threadIdx.x;
-  float td[K];
-  int ti[K];
-#pragma unroll
-  for (int i = 0; i < K; ++i) { td[i] = FLT_MAX; ti[i] = -1; }
-  const size_t base = (size_t)q * nblk * K;
-  for (int c = tid; c < nblk * K; c += 256) {
-    const float v = ws_d[base + c];
-    if (v < td[K - 1]) topk_insert<K>(td, ti, v, ws_i[base + c]);
-  }
-  if (tid == 0) {
-    float s = 0.f;
-    if (!IP && qnorm_src)
-      for (int c = 0; c < d; ++c) s += qnorm_src[(size_t)q * d + c] * qnorm_src[(size_t)q * d + c];
-    qn = s;
-  }
-  block_select_topk<K, 256>(td, ti, sd, si, topk_smem + K * 8);
-  if (tid < k_out) {
-    const float v = sd[tid];
-    const int id = si[tid];
-    const bool valid = id >= 0 && v != FLT_MAX;
-    out_d[(size_t)q * k_out + tid] = valid ? (IP ? -v : v + qn) : (IP ? -FLT_MAX : FLT_MAX);
-    out_i[(size_t)q * k_out + tid] = valid ? (idmap ? idmap[id] : (int64_t)id) + id_offset : -1;
-  }
+// ---- selection by 64-bit keys (order image of the distance, id): keys order as (distance, id)
+// does, ids compared unsigned, so any order of arrival selects the same candidates
+typedef unsigned long long u64;
+constexpr int kCandBuf = 1024;   // candidates a workgroup holds
+
+__device__ __forceinline__ u64 cand_key(float v, uint32_t id) { return ((u64)fkey(v) << 32) | id; }
+__device__ __forceinline__ float key_value(u64 k) {
+  const uint32_t t = (uint32_t)(k >> 32);
+  return __uint_as_float((t & 0x80000000u) ? (t & 0x7fffffffu) : ~t);
 }
 
-constexpr size_t topk_merge_lds(int K) { return (size_t)K * 8 + topk_select_lds(K); }
+// buf[0, n) of kCandBuf unique keys -> its K least in ascending order at buf[0, min(n, K)).  Few
+// entries: every entry counts those below it; many: bitonic sort.  All 256 threads call it.
+__device__ __forceinline__ void keep_best(u64* buf, int n, int K) {
+  const int tid = threadIdx.x;
+  if (n <= 256) {
+    const u64 mine = tid < n ? buf[tid] : ~0ull;
+    int r = 0;
+    for (int j = 0; j < n; ++j) r += buf[j] < mine;
+    __syncthreads();
+    if (tid < n && r < K) buf[r] = mine;
+    __syncthreads();
+    return;
+  }
+  int P = 512;
+  while (P < n) P <<= 1;
+  for (int i = n + tid; i < P; i += 256) buf[i] = ~0ull;
+  __syncthreads();
+  for (int k = 2; k <= P; k <<= 1)
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      for (int i = tid; i < P / 2; i += 256) {
+        const int a = 2 * i - (i & (j - 1)), b = a + j;
+        const u64 x = buf[a], y = buf[b];
+        if ((x > y) == ((a & k) == 0)) { buf[a] = y; buf[b] = x; }
+      }
+      __syncthreads();
+    }
+}
+
+// Of the 256 threads' values, each the least of a share of its own: the K-th least (K <= 256),
+// which bounds the K-th least of all shares from above; FLT_MAX where fewer threads have one.
+// tm: 256 floats of LDS, 16-byte aligned.  All 256 threads call it.
+__device__ __forceinline__ float bound_of_minima(float mine, int K, float* tm, float* out) {
+  const int tid = threadIdx.x;
+  tm[tid] = mine;
+  if (tid == 0) *out = FLT_MAX;
+  __syncthreads();
+  int r = 0;
+  for (int j = 0; j < 256; j += 4) {
+    const float4 o = *reinterpret_cast<const float4*>(tm + j);
+    r += (o.x < mine || (o.x == mine && j < tid)) + (o.y < mine || (o.y == mine && j + 1 < tid)) +
+         (o.z < mine || (o.z == mine && j + 2 < tid)) + (o.w < mine || (o.w == mine && j + 3 < tid));
+  }
+  if (r == K - 1) *out = mine;
+  __syncthreads();
+  return *out;
+}
+
+// Merge a query's partial lists: ws_d / ws_i [nq][cnt], any order, FLT_MAX where nothing is; ids
+// are positions that idmap translates to stored 64-bit ids.  Grid: queries.  The bound of the
+// threads' minima leaves little more than k_out entries to order (64 lists of 64: 89 us as a
+// bisection over 64 registers a thread, 6 us so).
+static __global__ __launch_bounds__(256) void topk_merge_kernel(const float* __restrict__ ws_d, const int* __restrict__ ws_i,
+                                                                int cnt, int k_out, float* __restrict__ out_d,
+                                                                int64_t* __restrict__ out_i,
+                                                                const int64_t* __restrict__ idmap) {
+  __shared__ u64 buf[kCandBuf];
+  __shared__ __attribute__((aligned(16))) float tm[256];
+  __shared__ float s_b;
+  __shared__ int s_n;
+  const int q = blockIdx.x, tid = threadIdx.x;
+  const float* dq = ws_d + (size_t)q * cnt;
+  const int* iq = ws_i + (size_t)q * cnt;
+  float mine = FLT_MAX;
+  for (int c = tid; c < cnt; c += 256) mine = fminf(mine, dq[c]);
+  if (tid == 0) s_n = 0;
+  float most = bound_of_minima(mine, k_out, tm, &s_b);
+  for (int c = tid; c < cnt; c += 256) {
+    const float v = dq[c];
+    if (v <= most && v < FLT_MAX) {
+      const int at = atomicAdd(&s_n, 1);
+      if (at < kCandBuf) buf[at] = cand_key(v, (uint32_t)iq[c]);
+    }
+  }
+  __syncthreads();
+  int n = s_n;
+  if (n > kCandBuf) {            // equal distances by the thousand: in parts
+    __syncthreads();
+    n = 0;
+    u64 bound = cand_key(most, 0xffffffffu);
+    for (int c0 = 0; c0 < cnt; c0 += 256) {
+      if (tid == 0) s_n = n;
+      __syncthreads();
+      const float v = c0 + tid < cnt ? dq[c0 + tid] : FLT_MAX;
+      if (v < FLT_MAX) {
+        const u64 key = cand_key(v, (uint32_t)iq[c0 + tid]);
+        if (key <= bound) buf[atomicAdd(&s_n, 1)] = key;
+      }
+      __syncthreads();
+      n = s_n;
+      if (n > kCandBuf - 256) {
+        keep_best(buf, n, k_out);
+        n = k_out;
+        bound = buf[k_out - 1];
+      }
+      __syncthreads();
+    }
+  }
+  keep_best(buf, n, k_out);
+  if (tid < k_out) {
+    const bool ok = tid < n;
+    const u64 key = ok ? buf[tid] : 0;
+    out_d[(size_t)q * k_out + tid] = ok ? key_value(key) : FLT_MAX;
+    out_i[(size_t)q * k_out + tid] = ok ? idmap[(uint32_t)key] : -1;
+  }
+}
 
 }  // namespace docqa

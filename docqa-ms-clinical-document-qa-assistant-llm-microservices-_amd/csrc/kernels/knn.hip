@@ -18,52 +18,18 @@
 // Batches whose distances exceed the workspace run in pieces: queries are independent, row
 // pieces carry their K best along as (distance, row) pairs.
 #include "docqa_dist.h"
+#include "docqa_topk.h"
 
 using namespace docqa;
 
 namespace {
 
-typedef unsigned long long u64;
 constexpr int kMaxK = 64;
-constexpr int kBuf = 1024;      // candidates held
 constexpr int kTiles = 1024;    // tile list
-
-__device__ __forceinline__ u64 cand_key(float v, uint32_t row) {
-  const uint32_t b = __float_as_uint(v);
-  return ((u64)((b & 0x80000000u) ? ~b : (b | 0x80000000u)) << 32) | row;
-}
-__device__ __forceinline__ float key_value(u64 k) {
-  const uint32_t t = (uint32_t)(k >> 32);
-  return __uint_as_float((t & 0x80000000u) ? (t & 0x7fffffffu) : ~t);
-}
-
-// buf[0, n) -> its K least in ascending order at buf[0, min(n, K)).  Few entries: every entry
-// counts those below it; many: bitonic sort.  All 256 threads call it.
-__device__ void keep_best(u64* buf, int n, int K) {
-  const int tid = threadIdx.x;
-  if (n <= 256) {
-    const u64 mine = tid < n ? buf[tid] : ~0ull;
-    int r = 0;
-    for (int j = 0; j < n; ++j) r += buf[j] < mine;      // keys are unique: rows are
-    __syncthreads();
-    if (tid < n && r < K) buf[r] = mine;
-    __syncthreads();
-    return;
-  }
-  int P = 512;
-  while (P < n) P <<= 1;
-  for (int i = n + tid; i < P; i += 256) buf[i] = ~0ull;
-  __syncthreads();
-  for (int k = 2; k <= P; k <<= 1)
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      for (int i = tid; i < P / 2; i += 256) {
-        const int a = 2 * i - (i & (j - 1)), b = a + j;
-        const u64 x = buf[a], y = buf[b];
-        if ((x > y) == ((a & k) == 0)) { buf[a] = y; buf[b] = x; }
-      }
-      __syncthreads();
-    }
-}
+// up to here, and where tile minima do not single tiles out (T <= 4 K), a query's workgroup reads
+// every distance: 32 tiles, K 64: 156 -> 10 us a launch of 64 queries; 83 tiles, K 3 takes 9.7 us
+// from the minima and 12.7 us so
+constexpr int kFewTiles = 128;
 
 // One query's K best of a piece of rows [row0, row0 + 32 T) and of those carried from earlier
 // pieces.  Grid: queries.
@@ -73,21 +39,23 @@ __global__ __launch_bounds__(256) void knn_select_kernel(const float* __restrict
                                                          const float* __restrict__ xq, int d, bool ip,
                                                          float* __restrict__ out_d, int64_t* __restrict__ out_i,
                                                          int64_t id_offset) {
-  __shared__ u64 buf[kBuf];
+  __shared__ u64 buf[kCandBuf];
   __shared__ int list[kTiles];
   __shared__ __attribute__((aligned(16))) float tm[256];
   __shared__ int s_n, s_t;
-  __shared__ u64 s_bound;
-  __shared__ float s_qn[4];
+  __shared__ float s_qn[4], s_b;
   const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const float* mq = mins + (size_t)q * ldt;
+  // few tiles: the bound comes from the distances themselves, each thread's share of them; many:
+  // from the tiles' minima
+  const bool few = T <= kFewTiles && T <= 4 * K;
+  auto dist_at = [&](int e) { return D[((size_t)(e >> 5) * nq + q) * 32 + (e & 31)]; };
   float mine = FLT_MAX;
-  for (int t = tid; t < T; t += 256) mine = fminf(mine, mq[t]);
-  tm[tid] = mine;
-  if (tid == 0) {
-    s_bound = cand_key(FLT_MAX, 0);                      // below it: a value that is there
-    s_t = 0;
-  }
+  if (few)
+    for (int e = tid; e < T * 32; e += 256) mine = fminf(mine, dist_at(e));
+  else
+    for (int t = tid; t < T; t += 256) mine = fminf(mine, mq[t]);
+  if (tid == 0) s_t = 0;
   if (wave == 0) {                                       // carried keys: ascending, ~0 where there are fewer
     const u64 key = !first && lane < K ? carry[(size_t)q * K + lane] : ~0ull;
     buf[lane] = key;
@@ -100,29 +68,37 @@ __global__ __launch_bounds__(256) void knn_select_kernel(const float* __restrict
     s = wave_sum(s);
     if (lane == 0) s_qn[wave] = s;
   }
-  __syncthreads();
-  // the bound: the K-th least of the threads' minima, each of a tile of its own
-  int r = 0;
-  for (int j = 0; j < 256; j += 4) {
-    const float4 o = *reinterpret_cast<const float4*>(tm + j);
-    r += (o.x < mine || (o.x == mine && j < tid)) + (o.y < mine || (o.y == mine && j + 1 < tid)) +
-         (o.z < mine || (o.z == mine && j + 2 < tid)) + (o.w < mine || (o.w == mine && j + 3 < tid));
-  }
-  if (r == K - 1 && mine < FLT_MAX) s_bound = cand_key(mine, 0xffffffffu);
-  __syncthreads();
+  float most = bound_of_minima(mine, K, tm, &s_b);
   int n = s_n;                                           // candidates held (uniform)
-  u64 bound = min(s_bound, buf[K - 1]);                  // carried rows are the lower ones: ties are theirs
-  // tiles within the bound; a list that overflows (equal rows by the thousand) is taken in parts
-  float most = key_value(bound);
-  int step = T;
-  for (int t = tid; t < T; t += 256)
-    if (mq[t] <= most && mq[t] < FLT_MAX) {
-      const int at = atomicAdd(&s_t, 1);
-      if (at < kTiles) list[at] = t;
+  u64 bound = min(cand_key(most, 0xffffffffu), buf[K - 1]);   // carried rows are the lower ones: ties are theirs
+  most = fminf(most, key_value(buf[K - 1]));
+  bool done = false;
+  if (few) {
+    for (int e = tid; e < T * 32; e += 256) {
+      const float v = dist_at(e);
+      const u64 key = cand_key(v, row0 + (uint32_t)e);
+      if (v < FLT_MAX && key < bound) {
+        const int at = atomicAdd(&s_n, 1);
+        if (at < kCandBuf) buf[at] = key;
+      }
     }
+    __syncthreads();
+    done = s_n <= kCandBuf;
+    if (done) n = s_n;
+    __syncthreads();
+    if (!done && tid == 0) s_n = n;                      // equal rows by the hundred: the general way
+  }
+  // tiles within the bound; a list that overflows (equal rows by the thousand) is taken in parts
+  int step = T;
+  if (!done)
+    for (int t = tid; t < T; t += 256)
+      if (mq[t] <= most && mq[t] < FLT_MAX) {
+        const int at = atomicAdd(&s_t, 1);
+        if (at < kTiles) list[at] = t;
+      }
   __syncthreads();
   if (s_t > kTiles) step = kTiles;
-  for (int t0 = 0; t0 < T; t0 += step) {
+  for (int t0 = 0; t0 < T && !done; t0 += step) {
     if (step != T) {
       __syncthreads();
       if (tid == 0) s_t = 0;
@@ -143,7 +119,7 @@ __global__ __launch_bounds__(256) void knn_select_kernel(const float* __restrict
       __syncthreads();
       n = s_n;
       __syncthreads();                                   // (read by all before the next group counts on)
-      if (n > kBuf - 256) {
+      if (n > kCandBuf - 256) {
         keep_best(buf, n, K);
         n = K;                                           // (n > K here)
         bound = buf[K - 1];

@@ -54,14 +54,15 @@ def pca_rotation(x: torch.Tensor, M: int) -> torch.Tensor:
 
 
 def probes_per_workgroup(nq: int, nprobe: int) -> int:
-    """Probed lists per scan workgroup: enough workgroups to fill the chip several times
-    over (~4096: two 57 KB-LDS workgroups per CU x 256 CUs x 8 rounds) without re-loading
-    each query's 48 KB LUT for only a list or two (DOCQA_IVFPQ_PC overrides)."""
+    """Probed lists per scan workgroup: about 4096 workgroups, but as each loads the query's 48 KB
+    LUT first, four lists each where that leaves 1024 (three fit a CU's LDS at M = 96).  us a search,
+    1 / 4 / 8 / 16 lists: 64 queries x 64 probes 143 / 131 / 127 / 157, 16 x 32 75 / 89 / 110 / 147,
+    256 x 256 1217 / 917 / 855 / 802.  DOCQA_IVFPQ_PC overrides."""
     env = os.environ.get("DOCQA_IVFPQ_PC")
     if env:
         return max(1, int(env))
     chunks = max(1, min(nprobe, -(-4096 // max(1, nq))))
-    return -(-nprobe // chunks)
+    return max(-(-nprobe // chunks), min(4, nq * nprobe // 1024))
 
 
 # auto scan: above this E||c||^2 / E||r^||^2 the exact-fp32 LUT kernel is used
@@ -92,6 +93,32 @@ class IVFPQIndex:
         # a FAISS load, which stores no such term
         self.norms: torch.Tensor | None = torch.empty(0, dtype=torch.float32, device=self.device)
         self.ntotal = 0
+
+    # what searches derive from the quantizers is made once per assignment of them (train, a load,
+    # a move to another device)
+    @property
+    def centroids(self) -> torch.Tensor | None:
+        return self._centroids
+
+    @centroids.setter
+    def centroids(self, t: torch.Tensor | None) -> None:
+        self._centroids, self._cnorm, self._auto_mode = t, None, None
+
+    @property
+    def pq(self) -> torch.Tensor | None:
+        return self._pq
+
+    @pq.setter
+    def pq(self, t: torch.Tensor | None) -> None:
+        self._pq, self._auto_mode = t, None
+
+    @property
+    def cnorm(self) -> torch.Tensor:
+        """Squared norms of the coarse centroids."""
+        n = self._cnorm
+        if n is None:
+            n = self._cnorm = ops.row_norms(self.centroids)
+        return n
 
     @property
     def is_trained(self) -> bool:
@@ -185,7 +212,7 @@ class IVFPQIndex:
     def search(self, xq, k: int, nprobe: int | None = None):
         nprobe = min(nprobe or self.nprobe, self.nlist)
         xq = self._in(xq).contiguous()
-        cn = (self.centroids ** 2).sum(1)
+        cn = self.cnorm
         if nprobe <= 64 and self.device.type == "cuda":
             _, probes = ops.knn(self.centroids, cn, xq, nprobe, False, 0)
         else:   # wide probes (the 10M operating points: nprobe 128..512): coarse.hip
@@ -211,11 +238,10 @@ class IVFPQIndex:
         mode = os.environ.get("DOCQA_IVFPQ_SCAN", "auto")
         if mode in ("pt", "lut"):
             return mode
-        if getattr(self, "_auto_src", None) is not (self.centroids, self.pq):
+        if self._auto_mode is None:
             cn = float((self.centroids.float() ** 2).sum(1).mean())
             rn = float((self.pq.float() ** 2).sum(-1).mean(1).sum())      # E||r^||^2 over the M sub-spaces
             self._auto_mode = "lut" if cn > _PT_MAX_RATIO * max(rn, 1e-30) else "pt"
-            self._auto_src = (self.centroids, self.pq)
         return self._auto_mode
 
     def _search_reference(self, xq, probes, k):

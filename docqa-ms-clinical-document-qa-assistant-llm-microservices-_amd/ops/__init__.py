@@ -1710,6 +1710,13 @@ def fp32_matmul_nt(x, w):
     return x.float() @ w.float().t()
 
 
+def row_norms(x):
+    """Squared norms fp32 [n] of the rows of fp32 ``x`` [n, d]."""
+    if _gpu(x):
+        return _native().row_norms(x.contiguous())
+    return (x ** 2).sum(1)
+
+
 def coarse_probes(xq, centroids, cnorm, nprobe: int):
     """IVF coarse quantizer: int64 [nq, nprobe] nearest centroids by squared L2, ascending,
     ties to the lower centroid id.  GPU: csrc/kernels/coarse.hip (MFMA fp32 distances +

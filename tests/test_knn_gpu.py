@@ -81,3 +81,41 @@ def test_fp32_product(n, nq, d):
     got = ops.fp32_matmul_nt(x, w).double()
     ref = x.double() @ w.double().T
     assert (got - ref).abs().max() <= 2.0 ** -22 * d ** 0.5 * float(x.norm(dim=1).max() * w.norm(dim=1).max())
+
+
+def test_ivfpq_equal_distances_by_the_thousand():
+    """Every stored vector at one distance: partial lists whose merge holds more equal entries
+    than its buffer still give k different vectors."""
+    from docqa_amd.index.ivfpq import IVFPQIndex
+
+    idx = IVFPQIndex(64, 64, 16, device="cuda")
+    idx.centroids, idx.pq = torch.zeros(64, 64, device="cuda"), torch.zeros(16, 256, 4, device="cuda")
+    n = 64 * 100
+    idx.codes = torch.randint(0, 256, (n, 16), device="cuda", dtype=torch.uint8)
+    idx.ids, idx.ntotal = torch.arange(n, device="cuda") + 5, n
+    idx.list_off = torch.arange(65, device="cuda") * 100
+    q = torch.randn(3, 64, device="cuda")
+    for k in (1, 64):
+        D, I = idx.search(q, k, nprobe=64)
+        assert (D - (q ** 2).sum(1, keepdim=True)).abs().max() < 1e-3       # fp16 tables of zeros: fp32 rounding
+        assert all(len(set(r)) == k and min(r) >= 5 and max(r) < n + 5 for r in I.tolist())
+
+
+@pytest.mark.parametrize("d,dtype", [(37, torch.float32), (64, torch.float32), (768, torch.bfloat16), (10, torch.bfloat16)])
+@pytest.mark.parametrize("metric", ["l2", "ip"])
+def test_refine_widths(d, dtype, metric):
+    from docqa_amd.index.refine import RefineFlat
+
+    x = torch.randn(500, d, device="cuda").to(dtype)
+    q = torch.randn(5, d, device="cuda")
+    cand = torch.stack([torch.randperm(500, device="cuda")[:57] for _ in range(5)])
+    cand[:, 3] = -1
+    D, I = ops._native().refine_flat(x, q, cand, 9, metric == "ip")
+    D2, I2 = RefineFlat(None, x, metric).rerank(q, cand, 9)
+    # (sums of d products in another order; random distances are further apart than that)
+    assert torch.equal(I, I2) and torch.allclose(D, D2, rtol=1e-4, atol=1e-4)
+
+
+def test_row_norms():
+    x = torch.randn(1001, 37, device="cuda")
+    assert torch.allclose(ops.row_norms(x), (x ** 2).sum(1), rtol=1e-5)
