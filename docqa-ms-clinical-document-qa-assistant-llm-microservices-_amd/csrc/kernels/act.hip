@@ -14,7 +14,6 @@
 using namespace docqa;
 
 __device__ __forceinline__ float silu(float x) { return x / (1.f + __expf(-x)); }
-__device__ __forceinline__ float gelu_erf(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752f)); }
 
 // IL: gate|up rows interleaved in blocks of 8 (the layout the decode GEMM's fused SwiGLU
 // epilogue reads): output chunk c = silu(chunk 2c) * chunk 2c+1 of the row.

@@ -6,7 +6,8 @@
 // GEMM with its bias+GELU, the QKV and output projections with their biases, so no
 // separate element-wise pass re-reads the [tokens, 4H] activations from HBM.
 //
-// Structure (cdna_hip_programming.md §5 "canonical CDNA GEMM", T1, T2, T14):
+// Structure of the 128 x 128 kernel (cdna_hip_programming.md §5 "canonical CDNA GEMM", T1, T2, T14);
+// gemm_ring_kernel below is the one for large row counts:
 //   * 128x128 block tile, BK = 64, 4 waves in 2x2, each wave a 64x64 sub-tile of
 //     4x4 v_mfma_f32_16x16x32_bf16 accumulators (64 fp32 registers);
 //   * A and W tiles are both row-major [row][k] in LDS (W^T's k-contiguous rows are
@@ -19,6 +20,7 @@
 //   * epilogue through LDS: accumulators -> fp32 tile -> coalesced 16-B rows with the
 //     bias / GELU / residual applied once per output element.
 // Shapes: N % 128 == 0, K % 64 == 0, any M.
+#include "docqa_asm.h"
 #include "docqa_common.h"
 
 using namespace docqa;
@@ -31,10 +33,6 @@ enum Epi { EPI_NONE = 0, EPI_BIAS = 1, EPI_BIAS_GELU = 2, EPI_BIAS_RES = 3, EPI_
 
 __device__ __forceinline__ int sw_off(int row, int ch) {  // element offset in a [128][64] tile
   return row * BK + ((ch ^ ((row >> 1) & 7)) << 3);
-}
-
-__device__ __forceinline__ float gelu_erf(float x) {
-  return 0.5f * x * (1.f + erff(x * 0.70710678118654752f));
 }
 
 template <int EPI>
@@ -172,6 +170,172 @@ __global__ __launch_bounds__(256) void gemm_kernel(const uint16_t* __restrict__ 
     }
   }
 }
+
+// ---- 256 rows x 128 columns a workgroup, two workgroups a CU: row counts that fill the chip.
+// The 128 x 128 kernel reads 64 KB of LDS for 512 clocks of MFMA a K-step and is bound by that
+// (bge-base, 30720 rows, us of QKV / O / FFN up / down: 146 / 54 / 226 / 173; here 119 / 49 / 175 /
+// 140, 0.9 to 1.05 PFLOP/s, the matrix cores busy 45 % of the time at the 1.9 GHz this load runs at,
+// the rest in the latency of units and epilogues).
+// Here a wave owns 128 rows x 64 columns (v_mfma_f32_32x32x16_bf16: 48 KB for 1024 clocks), and a
+// workgroup's epilogue runs under the other one's products.
+//   * K-tiles of 64 come as three units of 128 rows x 64 (whole 128-byte lines: with 64-byte rows
+//     LDS-DMA moves 15 TB/s over the chip, with 128-byte ones 20 to 29) through a ring of five:
+//       HA0 = the first 64 rows of both wave rows, HB = the columns, HA1 = the last 64 rows
+//     phase 1 of K-tile t reads units 3t (HA0) and 3t + 1 (HB, kept in registers), phase 2 reads
+//     3t + 2 (HA1); phase 1 issues unit 3t + 4 over 3t - 1, phase 2 issues 3t + 5 and 3t + 6 over
+//     3t and 3t + 1, each read by every wave before the barrier that opens the phase.  At that
+//     barrier two units are in flight (vmcnt(8)), two phases ahead of their reads;
+//   * the MFMA's row operand is W, its column operand A: a lane holds one output row and four
+//     neighbouring columns per register quad, 8-byte pieces of the bf16 tile;
+//   * the tile is put together in LDS (16-B chunk ^ (row & 15): 32 rows' pieces hit distinct
+//     banks) and stored in whole rows; the residual comes into the same places by LDS-DMA first
+//     and is added in fp32 before the one rounding.
+constexpr int WM = 256, WN = 128;
+constexpr int UNIT = 128 * BK * 2, NUNIT = 5;         // 16 KB units of the ring, 80 KB
+
+template <int EPI>
+__global__ __launch_bounds__(256, 2) void gemm_ring_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ W,
+                                                           const uint16_t* __restrict__ bias,
+                                                           const uint16_t* __restrict__ res, uint16_t* __restrict__ C,
+                                                           int M, int N, int K) {
+  __shared__ __attribute__((aligned(16))) char smem[NUNIT * UNIT];
+  static_assert(NUNIT * UNIT >= WM * WN * 2, "epilogue tile");
+  const int nbn = N / WN;
+  const int wg = xcd_remap(blockIdx.x, gridDim.x);
+  const int row0 = (wg / nbn) * WM, col0 = (wg % nbn) * WN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = wave & 1, wc = wave >> 1;
+  const int l32 = lane & 31, hh = lane >> 5;
+  const uint32_t lds = lds_u32(smem);
+
+  // four 16-B pieces a thread and unit: unit rows 32 i + tid / 8
+  const char* ab = (const char*)(A + (size_t)row0 * K);
+  const char* wb = (const char*)(W + (size_t)col0 * K);
+  const uint32_t lch = (uint32_t)((tid & 7) ^ ((tid >> 4) & 7)) * 16;     // (row >> 1) & 7 is the thread's own
+  uint32_t aoff[2][4], boff[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = i * 32 + (tid >> 3);
+    boff[i] = (uint32_t)r * (uint32_t)(K * 2) + lch;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      aoff[h][i] = (uint32_t)min((r >> 6) * 128 + h * 64 + (r & 63), M - 1 - row0) * (uint32_t)(K * 2) + lch;
+  }
+  // unit `part` (0 HA0, 1 HB, 2 HA1) of K-tile kt into ring slot `slot`
+  auto issue = [&](int part, int kt, int slot) {
+    const uint32_t d = lds + (uint32_t)(slot * UNIT + wave * 1024);
+    const uint32_t k = (uint32_t)kt * (BK * 2);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      glds16_off(part == 1 ? wb : ab, (part == 1 ? boff[i] : aoff[part >> 1][i]) + k,
+                 __builtin_amdgcn_readfirstlane(d + i * 4096));
+  };
+  auto open = [&]() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    ring_barrier();
+  };
+  // 16-B chunk `ch` of unit row `row`: 32-row fragment reads hit distinct banks
+  auto frag = [&](int slot, int row, int ch) {
+    return *reinterpret_cast<const bf16x8*>(smem + slot * UNIT + row * 128 + ((ch ^ ((row >> 1) & 7)) << 4));
+  };
+
+  f32x16 acc[2][4];
+#pragma unroll
+  for (int n = 0; n < 2; ++n)
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[n][m][r] = 0.f;
+  bf16x8 w[4][2];                                    // [16-deep k-step][n-tile] of the current K-tile
+  auto phase = [&](int slot_a, int slot_b, bool first) {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      if (first) {
+#pragma unroll
+        for (int n = 0; n < 2; ++n) w[ks][n] = frag(slot_b, wc * 64 + n * 32 + l32, ks * 2 + hh);
+      }
+      bf16x8 a[2];
+#pragma unroll
+      for (int m = 0; m < 2; ++m) a[m] = frag(slot_a, wr * 64 + m * 32 + l32, ks * 2 + hh);
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+          f32x16& c = acc[n][first ? m : 2 + m];
+          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[ks][n], a[m], c, 0, 0, 0);
+        }
+    }
+  };
+
+  const int nk = K / BK;
+  issue(0, 0, 0);
+  issue(1, 0, 1);
+  issue(2, 0, 2);
+  if (nk > 1) issue(0, 1, 3);
+  int s0 = 0;                                        // slot of unit 3t
+  auto slot = [&](int k) { return s0 + k < NUNIT ? s0 + k : s0 + k - NUNIT; };   // of unit 3t + k, k <= 4
+  for (int t = 0; t < nk - 1; ++t) {
+    wait_vmcnt<8>();
+    open();
+    issue(1, t + 1, slot(4));
+    phase(slot(0), slot(1), true);
+    wait_vmcnt<8>();
+    open();
+    issue(2, t + 1, slot(0));
+    if (t + 2 < nk) issue(0, t + 2, slot(1));
+    phase(slot(2), 0, false);
+    s0 = slot(3);
+  }
+  wait_vmcnt<4>();
+  open();
+  phase(slot(0), slot(1), true);
+  wait_vmcnt<0>();
+  open();
+  phase(slot(2), 0, false);
+  open();                                            // the ring is the epilogue's tile now
+
+  // 16-B chunk of the tile that piece `it` of this thread is: row 16 it + tid / 16
+  const int prow = tid >> 4, pcol = ((tid & 15) ^ prow) * 8;
+  if constexpr (EPI == EPI_BIAS_RES) {
+    const char* rb = (const char*)(res + (size_t)row0 * N + col0);
+#pragma unroll
+    for (int it = 0; it < 16; ++it)
+      glds16_off(rb, (uint32_t)min(16 * it + prow, M - 1 - row0) * (uint32_t)(N * 2) + pcol * 2,
+                 __builtin_amdgcn_readfirstlane(lds + it * 4096 + wave * 1024));
+    wait_vmcnt<0>();
+    ring_barrier();
+  }
+#pragma unroll
+  for (int n = 0; n < 2; ++n)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int col = wc * 64 + n * 32 + 8 * g + 4 * hh;
+      float b[4] = {0.f, 0.f, 0.f, 0.f};
+      if constexpr (EPI != EPI_NONE) add4(b, *reinterpret_cast<const uint2*>(bias + col0 + col));
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const int row = wr * 128 + m * 32 + l32;
+        uint2* at = reinterpret_cast<uint2*>(smem + row * 256 + (((col >> 3) ^ (row & 15)) << 4) + (hh << 3));
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = acc[n][m][4 * g + e] + b[e];
+        if constexpr (EPI == EPI_BIAS_GELU) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = gelu_erf(v[e]);
+        }
+        if constexpr (EPI == EPI_BIAS_RES) add4(v, *at);
+        *at = make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
+      }
+    }
+  __syncthreads();
+  uint16_t* out = C + (size_t)row0 * N + col0 + pcol;
+#pragma unroll
+  for (int it = 0; it < 16; ++it) {
+    const int r = 16 * it + prow;
+    const uint4 v = *reinterpret_cast<const uint4*>(smem + it * 4096 + tid * 16);
+    if (row0 + r < M) *reinterpret_cast<uint4*>(out + (size_t)r * N) = v;
+  }
+}
 }  // namespace
 
 int docqa_gemm(const void* A, const void* W, const void* bias, const void* res, void* C, int M,
@@ -184,6 +348,20 @@ int docqa_gemm(const void* A, const void* W, const void* bias, const void* res, 
   const uint16_t *a = (const uint16_t*)A, *w = (const uint16_t*)W, *b = (const uint16_t*)bias,
                  *r = (const uint16_t*)res;
   uint16_t* c = (uint16_t*)C;
+  // from 256 tiles of 256 x 128 on, a workgroup a CU (us, 128 x 128 / ring: bge QKV 4096 rows, 288
+  // tiles, 28.1 / 25.0, 30720 rows 146 / 119; FFN down, K 3072, 8192 rows, 192 tiles, 48.6 / 54.2,
+  // 19000 rows, 450 tiles, 103 / 91); row offsets inside a tile are 32-bit
+  if (epi != EPI_GLU && (long long)((M + WM - 1) / WM) * (N / WN) >= 256 && (long long)WM * (K > N ? K : N) * 2 < (1ll << 32)) {
+    const int wgs = (N / WN) * ((M + WM - 1) / WM);
+    switch (epi) {
+      case EPI_NONE: gemm_ring_kernel<EPI_NONE><<<wgs, 256, 0, s>>>(a, w, b, r, c, M, N, K); break;
+      case EPI_BIAS: gemm_ring_kernel<EPI_BIAS><<<wgs, 256, 0, s>>>(a, w, b, r, c, M, N, K); break;
+      case EPI_BIAS_GELU: gemm_ring_kernel<EPI_BIAS_GELU><<<wgs, 256, 0, s>>>(a, w, b, r, c, M, N, K); break;
+      default: gemm_ring_kernel<EPI_BIAS_RES><<<wgs, 256, 0, s>>>(a, w, b, r, c, M, N, K); break;
+    }
+    DOCQA_CHECK_LAUNCH();
+    return 0;
+  }
   switch (epi) {
     case EPI_NONE: gemm_kernel<EPI_NONE><<<nwg, 256, 0, s>>>(a, w, b, r, c, M, N, K); break;
     case EPI_BIAS: gemm_kernel<EPI_BIAS><<<nwg, 256, 0, s>>>(a, w, b, r, c, M, N, K); break;
