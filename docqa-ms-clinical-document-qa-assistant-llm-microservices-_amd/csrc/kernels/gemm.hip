@@ -336,6 +336,134 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(const uint16_t* __res
     if (row0 + r < M) *reinterpret_cast<uint4*>(out + (size_t)r * N) = v;
   }
 }
+
+// ---- few rows: T x T tiles, K split over the workgroup's 4 waves.  Such products are bound by
+// the latency of one K walk and by what a CU can fetch, so a workgroup keeps five 16 KB stages in
+// flight, and each wave multiplies its quarter of every stage (a fragment read feeds T / 32 MFMAs
+// where 2 x 2 waves would read twice as much); the four sums meet in LDS, and whole rows leave
+// with bias, GELU or residual applied in fp32.
+template <int T, int EPI>
+__global__ __launch_bounds__(256, 2) void gemm_few_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ W,
+                                                          const uint16_t* __restrict__ bias,
+                                                          const uint16_t* __restrict__ res, uint16_t* __restrict__ C,
+                                                          int M, int N, int K) {
+  constexpr int KB = 4096 / T;                       // k's of a stage: 16 KB of both operands
+  constexpr int ROWB = KB * 2, CPR = ROWB / 16;      // bytes and 16-B chunks of a stage row
+  constexpr int STAGE = 2 * T * ROWB, NS = 5, L = STAGE / 4096;
+  constexpr int TI = T / 32, KS = CPR / 8;           // MFMA tiles a side, 16-deep k-steps a wave and stage
+  constexpr int PITCH = T + 4;
+  __shared__ __attribute__((aligned(16))) char smem[NS * STAGE];
+  static_assert(4 * T * PITCH * 4 <= NS * STAGE, "partial sums");
+  const int nbn = N / T;
+  const int wg = xcd_remap(blockIdx.x, gridDim.x);
+  const int row0 = (wg / nbn) * T, col0 = (wg % nbn) * T;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hh = lane >> 5;
+  const uint32_t lds = lds_u32(smem);
+  // 16-B chunk `ch` of stage row `row`: 32-row fragment reads hit distinct banks
+  auto swz = [](int row, int ch) { return CPR == 8 ? ch ^ ((row >> 1) & 7) : ch ^ (row & 15); };
+
+  const char* ab = (const char*)(A + (size_t)row0 * K);
+  const char* wb = (const char*)(W + (size_t)col0 * K);
+  uint32_t off[L];
+#pragma unroll
+  for (int i = 0; i < L; ++i) {
+    const int r = (i * 256 + tid) / CPR, lr = r % T;               // rows of A, then of W
+    off[i] = (uint32_t)(r < T ? min(lr, M - 1 - row0) : lr) * (uint32_t)(K * 2) + swz(lr, tid % CPR) * 16;
+  }
+  auto stage = [&](int kt, int buf) {
+    const uint32_t d = lds + (uint32_t)(buf * STAGE + wave * 1024);
+#pragma unroll
+    for (int i = 0; i < L; ++i)
+      glds16_off(i < L / 2 ? ab : wb, off[i] + (uint32_t)kt * ROWB, __builtin_amdgcn_readfirstlane(d + i * 4096));
+  };
+
+  f32x16 acc[TI][TI];
+#pragma unroll
+  for (int n = 0; n < TI; ++n)
+#pragma unroll
+    for (int m = 0; m < TI; ++m)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[n][m][r] = 0.f;
+  const int nk = K / KB;
+#pragma unroll
+  for (int t = 0; t < NS - 1; ++t)
+    if (t < nk) stage(t, t);
+  int buf = 0;
+  for (int kt = 0; kt < nk; ++kt) {
+    // stage kt has landed: of the later ones up to NS - 2 may be in flight
+    const int later = min(NS - 2, nk - 1 - kt);
+    if (later == 3) wait_vmcnt<3 * L>();
+    else if (later == 2) wait_vmcnt<2 * L>();
+    else if (later == 1) wait_vmcnt<L>();
+    else wait_vmcnt<0>();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    ring_barrier();                                  // and every wave has read what the next issue overwrites
+    if (kt + NS - 1 < nk) stage(kt + NS - 1, buf ? buf - 1 : NS - 1);
+    const char* sa = smem + buf * STAGE;
+    const char* sw = sa + T * ROWB;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int ch = (wave * KS + ks) * 2 + hh;
+      bf16x8 a[TI], w[TI];
+#pragma unroll
+      for (int i = 0; i < TI; ++i) {
+        const int r = i * 32 + l32;
+        a[i] = *reinterpret_cast<const bf16x8*>(sa + r * ROWB + swz(r, ch) * 16);
+        w[i] = *reinterpret_cast<const bf16x8*>(sw + r * ROWB + swz(r, ch) * 16);
+      }
+#pragma unroll
+      for (int n = 0; n < TI; ++n)
+#pragma unroll
+        for (int m = 0; m < TI; ++m) acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[n], a[m], acc[n][m], 0, 0, 0);
+    }
+    buf = buf == NS - 1 ? 0 : buf + 1;
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  ring_barrier();                                    // the ring holds the partial sums now
+  float* part = reinterpret_cast<float*>(smem);
+#pragma unroll
+  for (int n = 0; n < TI; ++n)
+#pragma unroll
+    for (int m = 0; m < TI; ++m)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<f32x4*>(part + (wave * T + m * 32 + l32) * PITCH + n * 32 + 8 * g + 4 * hh) =
+            f32x4{acc[n][m][4 * g], acc[n][m][4 * g + 1], acc[n][m][4 * g + 2], acc[n][m][4 * g + 3]};
+  __syncthreads();
+  constexpr int TPR = T / 8, RPI = 256 / TPR;        // threads a row, rows a pass
+#pragma unroll
+  for (int it = 0; it < (T + RPI - 1) / RPI; ++it) {
+    const int r = it * RPI + tid / TPR, c = (tid % TPR) * 8;
+    if (r >= T || row0 + r >= M) break;
+    float v[8] = {};
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+#pragma unroll
+      for (int e = 0; e < 8; e += 4) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(part + (w * T + r) * PITCH + c + e);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[e + k] += x[k];
+      }
+    float b[8];
+    if constexpr (EPI != EPI_NONE) {
+      unpack8(*reinterpret_cast<const uint4*>(bias + col0 + c), b);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] += b[e];
+    }
+    if constexpr (EPI == EPI_BIAS_GELU) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = gelu_erf(v[e]);
+    }
+    const size_t at = (size_t)(row0 + r) * N + col0 + c;
+    if constexpr (EPI == EPI_BIAS_RES) {
+      unpack8(*reinterpret_cast<const uint4*>(res + at), b);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] += b[e];
+    }
+    *reinterpret_cast<uint4*>(C + at) = pack8(v);
+  }
+}
 }  // namespace
 
 int docqa_gemm(const void* A, const void* W, const void* bias, const void* res, void* C, int M,
@@ -348,19 +476,37 @@ int docqa_gemm(const void* A, const void* W, const void* bias, const void* res, 
   const uint16_t *a = (const uint16_t*)A, *w = (const uint16_t*)W, *b = (const uint16_t*)bias,
                  *r = (const uint16_t*)res;
   uint16_t* c = (uint16_t*)C;
-  // from 256 tiles of 256 x 128 on, a workgroup a CU (us, 128 x 128 / ring: bge QKV 4096 rows, 288
-  // tiles, 28.1 / 25.0, 30720 rows 146 / 119; FFN down, K 3072, 8192 rows, 192 tiles, 48.6 / 54.2,
-  // 19000 rows, 450 tiles, 103 / 91); row offsets inside a tile are 32-bit
-  if (epi != EPI_GLU && (long long)((M + WM - 1) / WM) * (N / WN) >= 256 && (long long)WM * (K > N ? K : N) * 2 < (1ll << 32)) {
-    const int wgs = (N / WN) * ((M + WM - 1) / WM);
-    switch (epi) {
-      case EPI_NONE: gemm_ring_kernel<EPI_NONE><<<wgs, 256, 0, s>>>(a, w, b, r, c, M, N, K); break;
-      case EPI_BIAS: gemm_ring_kernel<EPI_BIAS><<<wgs, 256, 0, s>>>(a, w, b, r, c, M, N, K); break;
-      case EPI_BIAS_GELU: gemm_ring_kernel<EPI_BIAS_GELU><<<wgs, 256, 0, s>>>(a, w, b, r, c, M, N, K); break;
-      default: gemm_ring_kernel<EPI_BIAS_RES><<<wgs, 256, 0, s>>>(a, w, b, r, c, M, N, K); break;
+  // by how the tiles fill the chip (us): 32 x 32 up to two workgroups a CU (32 / 64 wide: bge QKV 128
+  // rows, 288 workgroups, 5.7 / 6.3, 256 rows, 576 of them, 8.0 / 6.5), 64 x 64 up to three (64 / 128
+  // wide: QKV 1024 rows, 576, 13.6 / 14.4, 1500 rows, 864, 16.6 / 14.7; O 4096 rows, 768, 13.2 / 13.5),
+  // 256 x 128 from one on (128 wide / ring: QKV 4096 rows, 288, 28.1 / 25.0, 30720 rows 146 / 119;
+  // FFN down, K 3072, 8192 rows, 192, 48.6 / 54.2, 19000 rows, 450, 103 / 91).  Row offsets inside
+  // those tiles are 32-bit
+  auto tiles = [&](int tm, int tn) { return (long long)((M + tm - 1) / tm) * (N / tn); };
+#define DOCQA_GEMM_EPI(KERNEL, GRID)                                                             \
+  do {                                                                                           \
+    const int g_ = (int)(GRID);                                                                  \
+    if (epi == EPI_NONE) KERNEL(EPI_NONE)<<<g_, 256, 0, s>>>(a, w, b, r, c, M, N, K);            \
+    else if (epi == EPI_BIAS) KERNEL(EPI_BIAS)<<<g_, 256, 0, s>>>(a, w, b, r, c, M, N, K);       \
+    else if (epi == EPI_BIAS_GELU) KERNEL(EPI_BIAS_GELU)<<<g_, 256, 0, s>>>(a, w, b, r, c, M, N, K); \
+    else KERNEL(EPI_BIAS_RES)<<<g_, 256, 0, s>>>(a, w, b, r, c, M, N, K);                        \
+  } while (0)
+#define DOCQA_FEW32(E) gemm_few_kernel<32, E>
+#define DOCQA_FEW64(E) gemm_few_kernel<64, E>
+#define DOCQA_RING(E) gemm_ring_kernel<E>
+  if (epi < EPI_NONE || epi > EPI_GLU) return -1;
+  if (epi != EPI_GLU && (long long)WM * (K > N ? K : N) * 2 < (1ll << 32)) {
+    int kind = 0;
+    if (K % 128 == 0 && tiles(32, 32) <= 512) kind = 32;
+    else if (tiles(64, 64) <= 768) kind = 64;
+    else if (tiles(WM, WN) >= 256) kind = WM;
+    if (kind == 32) DOCQA_GEMM_EPI(DOCQA_FEW32, tiles(32, 32));
+    else if (kind == 64) DOCQA_GEMM_EPI(DOCQA_FEW64, tiles(64, 64));
+    else if (kind) DOCQA_GEMM_EPI(DOCQA_RING, tiles(WM, WN));
+    if (kind) {
+      DOCQA_CHECK_LAUNCH();
+      return 0;
     }
-    DOCQA_CHECK_LAUNCH();
-    return 0;
   }
   switch (epi) {
     case EPI_NONE: gemm_kernel<EPI_NONE><<<nwg, 256, 0, s>>>(a, w, b, r, c, M, N, K); break;
@@ -368,7 +514,6 @@ int docqa_gemm(const void* A, const void* W, const void* bias, const void* res, 
     case EPI_BIAS_GELU: gemm_kernel<EPI_BIAS_GELU><<<nwg, 256, 0, s>>>(a, w, b, r, c, M, N, K); break;
     case EPI_BIAS_RES: gemm_kernel<EPI_BIAS_RES><<<nwg, 256, 0, s>>>(a, w, b, r, c, M, N, K); break;
     case EPI_GLU: gemm_kernel<EPI_GLU><<<nwg, 256, 0, s>>>(a, w, b, r, c, M, N, K); break;
-    default: return -1;
   }
   DOCQA_CHECK_LAUNCH();
   return 0;

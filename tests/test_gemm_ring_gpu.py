@@ -1,5 +1,5 @@
-"""The encoder GEMM's 256 x 128 tiles (csrc/kernels/gemm.hip gemm_ring_kernel): K-tile counts around
-its ring, row remainders, every epilogue, against 64-bit products."""
+"""The encoder GEMM's tiles (csrc/kernels/gemm.hip): K-tile counts around their rings, row remainders,
+every epilogue, against 64-bit products."""
 import pytest
 import torch
 
@@ -11,9 +11,12 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [
     (256 * 128, 256, 64), (256 * 127 + 1, 256, 128), (256 * 85 + 255, 384, 192), (256 * 86 - 31, 384, 320),
     (256 * 28 + 129, 1152, 384), (256 * 14 + 37, 2304, 768), (256 * 43 + 5, 768, 3072),
+    # 32 x 32 and 64 x 64 tiles (K not a multiple of 128: the latter), 1 .. 6 stages, one row
+    (1, 128, 128), (24, 384, 256), (33, 1152, 384), (128, 768, 512), (31, 128, 640), (1, 128, 64), (65, 256, 192),
+    (300, 2304, 768), (1000, 768, 3072), (700, 3072, 320), (129, 128, 448),
 ])
 @pytest.mark.parametrize("epi", [ops.EPI_NONE, ops.EPI_BIAS, ops.EPI_BIAS_GELU, ops.EPI_BIAS_RES])
-def test_large_row_counts(M, N, K, epi):
+def test_products(M, N, K, epi):
     g = torch.Generator(device="cuda").manual_seed(M + K)
 
     def rnd(*s, std=1.0):
@@ -33,7 +36,7 @@ def test_large_row_counts(M, N, K, epi):
     assert (err <= 2.0 ** -8 * ref.abs() + 2.0 ** -18 * K ** 0.5).all()
 
 
-@pytest.mark.parametrize("M", [512, 256 * 129])      # the 128 x 128 tiles and the ring
+@pytest.mark.parametrize("M", [512, 12 * 1024, 256 * 129])      # 64 x 64, 128 x 128, ring
 def test_gelu_tails(M):
     """x Phi(x) keeps its relative precision where 1 + erf(x / sqrt 2) has lost it."""
     v = torch.linspace(-9, 9, M).to(torch.bfloat16)
