@@ -30,7 +30,7 @@ int docqa_decode_slots(const int* block_tables, int maxb, const int* positions, 
                        int* slots, int B, int BS, hipStream_t s);
 int docqa_decode_advance(const int64_t* nxt, int64_t* out, int* tokens, int* positions,
                          int* context_lens, const int* valid, int B, hipStream_t s);
-int docqa_bert_embed_ln(const int* ids, const int* pos, const int* tt, const void* wte,
+int docqa_bert_embed_ln(const int* ids, const int* pos, const int* cu, int B, const int* tt, const void* wte,
                         const void* wpe, const void* wtt, const void* g, const void* b, void* out,
                         int T, int H, float eps, hipStream_t s);
 int docqa_argmax(const void* logits, int rows, int V, int ld, int is_bf16, float* ws_v, int* ws_i,

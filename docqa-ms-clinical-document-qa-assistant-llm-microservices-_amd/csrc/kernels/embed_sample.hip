@@ -72,10 +72,24 @@ __global__ __launch_bounds__(256) void embed_rmsnorm_kernel(const int* __restric
   }
 }
 
+// Position of token t in its own sequence: the last of the B starts cu[0 .. B) that is <= t, found by a
+// wave that compares 64 starts at a time (two dependent loads up to 4096 sequences, none for one).
+__device__ __forceinline__ int packed_position(const int* __restrict__ cu, int B, int t, int lane) {
+  int lo = 0, n = B;
+  while (n > 1) {
+    const int step = (n + 63) >> 6, i = lane * step;
+    const int cnt = max(1, __popcll(__ballot(i < n && cu[lo + min(i, n - 1)] <= t)));
+    lo += (cnt - 1) * step;
+    n = min(step, n - (cnt - 1) * step);
+  }
+  return t - cu[lo];
+}
+
+// One wave a token.  Without `pos` the position comes from the sequence starts `cu`.
 template <int NV>
 __global__ __launch_bounds__(256) void bert_embed_ln_kernel(
-    const int* __restrict__ ids, const int* __restrict__ pos, const int* __restrict__ tt,
-    const uint16_t* __restrict__ wte, const uint16_t* __restrict__ wpe,
+    const int* __restrict__ ids, const int* __restrict__ pos, const int* __restrict__ cu, int B,
+    const int* __restrict__ tt, const uint16_t* __restrict__ wte, const uint16_t* __restrict__ wpe,
     const uint16_t* __restrict__ wtt, const uint16_t* __restrict__ gamma,
     const uint16_t* __restrict__ beta, uint16_t* __restrict__ out, int T, int H, float eps) {
   const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -83,7 +97,8 @@ __global__ __launch_bounds__(256) void bert_embed_ln_kernel(
   if (t >= T) return;
   const int nchunk = H >> 3;
   const uint4* w = reinterpret_cast<const uint4*>(wte + (size_t)ids[t] * H);
-  const uint4* p = reinterpret_cast<const uint4*>(wpe + (size_t)pos[t] * H);
+  const uint4* p =
+      reinterpret_cast<const uint4*>(wpe + (size_t)(pos ? pos[t] : packed_position(cu, B, t, lane)) * H);
   const uint4* y = reinterpret_cast<const uint4*>(wtt + (size_t)(tt ? tt[t] : 0) * H);
   float v[NV][8];
   float s = 0.f;
@@ -336,15 +351,16 @@ int docqa_embed_rmsnorm(const int* ids, const void* table, const void* w, void* 
   return 0;
 }
 
-int docqa_bert_embed_ln(const int* ids, const int* pos, const int* tt, const void* wte,
+int docqa_bert_embed_ln(const int* ids, const int* pos, const int* cu, int B, const int* tt, const void* wte,
                         const void* wpe, const void* wtt, const void* g, const void* b, void* out,
                         int T, int H, float eps, hipStream_t s) {
   if (T == 0) return 0;
+  if (!pos && (!cu || B < 1)) return -1;
   if (H % 8 != 0 || !docqa_aligned16(wte) || !docqa_aligned16(wpe) || !docqa_aligned16(wtt) ||
       !docqa_aligned16(g) || !docqa_aligned16(b) || !docqa_aligned16(out)) return -1;
   const int nv = (H / 8 + 63) / 64;
   dim3 grid((T + 3) / 4);
-#define BE(N) bert_embed_ln_kernel<N><<<grid, 256, 0, s>>>(ids, pos, tt, (const uint16_t*)wte, (const uint16_t*)wpe, (const uint16_t*)wtt, (const uint16_t*)g, (const uint16_t*)b, (uint16_t*)out, T, H, eps)
+#define BE(N) bert_embed_ln_kernel<N><<<grid, 256, 0, s>>>(ids, pos, cu, B, tt, (const uint16_t*)wte, (const uint16_t*)wpe, (const uint16_t*)wtt, (const uint16_t*)g, (const uint16_t*)b, (uint16_t*)out, T, H, eps)
   if (nv <= 1) BE(1); else if (nv <= 2) BE(2); else if (nv <= 4) BE(4); else return -1;
 #undef BE
   DOCQA_CHECK_LAUNCH();

@@ -24,6 +24,7 @@ from __future__ import annotations
 
 import math
 import os
+from array import array
 from dataclasses import dataclass
 
 import torch
@@ -142,6 +143,9 @@ class BertEncoder:
                       positions: torch.Tensor | None = None) -> torch.Tensor:
         """ids int32 [T] (packed), cu_seqlens int32 [B+1] -> last hidden [T, H] bf16."""
         cfg = self.cfg
+        if ops.bert_hidden_ok(cfg.hidden, cfg.intermediate, ids.shape[0], self.wte):
+            return ops.bert_hidden(ids, positions, cu_seqlens, max_len, self.wte, self.wpe, self.wtt, self.emb_g,
+                                   self.emb_b, self.layers, cfg.heads, self.scale, cfg.eps)
         if positions is None:
             positions = packed_positions(cu_seqlens, ids.shape[0])
         h = ops.bert_embed_ln(ids, positions, None, self.wte, self.wpe, self.wtt, self.emb_g,
@@ -182,9 +186,12 @@ def pack(token_lists: list[list[int]], max_seq_len: int, device) -> tuple[torch.
         flat.extend(t)
         cu.append(cu[-1] + len(t))
     max_len = max((cu[i + 1] - cu[i] for i in range(len(token_lists))), default=0)
-    ids = torch.tensor(flat, dtype=torch.int32).to(device, non_blocking=True)
-    cut = torch.tensor(cu, dtype=torch.int32).to(device, non_blocking=True)
-    return ids, cut, max_len
+    try:
+        both = torch.frombuffer(array("i", flat + cu), dtype=torch.int32)
+    except (TypeError, OverflowError):      # ids that are no whole numbers of 32 bits: torch's own conversion
+        both = torch.tensor(flat + cu, dtype=torch.int32)
+    both = both.to(device, non_blocking=True)       # one copy, two views
+    return both[:len(flat)], both[len(flat):], max_len
 
 
 class BertTokenClassifier(BertEncoder):

@@ -801,6 +801,22 @@ def bert_embed_ln(ids, pos, token_type, wte, wpe, wtt, gamma, beta, eps):
     return ref.bert_embed_ln(ids, pos, token_type, wte, wpe, wtt, gamma, beta, eps)
 
 
+BERT_LAYER = ("qkv_w", "qkv_b", "o_w", "o_b", "ln1_g", "ln1_b", "up_w", "up_b", "down_w", "down_b", "ln2_g", "ln2_b")
+
+
+def bert_hidden_ok(H: int, I: int, tokens: int, wte) -> bool:
+    """Whether :func:`bert_hidden` takes this stack: each of its products is one for the MFMA GEMM
+    (see :func:`linear_fused`); others go op by op."""
+    return _gpu(wte) and tokens > 0 and H % 128 == 0 and I % 128 == 0 and H <= 2048
+
+
+def bert_hidden(ids, positions, cu_seqlens, max_len, wte, wpe, wtt, gamma, beta, layers, heads: int, scale: float,
+                eps: float):
+    """Last hidden states [T, H] of a post-norm encoder, all of its launches from one call."""
+    return _native().bert_hidden(ids, positions, cu_seqlens, max_len, wte, wpe, wtt, gamma, beta,
+                                 [L[k] for L in layers for k in BERT_LAYER], heads, scale, eps)
+
+
 # ----------------------------------------------------------------------------- sampling
 def decode_slots(block_tables, positions, valid, BS: int):
     """Paged-cache slot of each decode row's next token, -1 for padded rows."""
