@@ -743,7 +743,8 @@ at::Tensor dgemm_glu(const at::Tensor& x, const at::Tensor& w) {
     CHECK_RC(docqa_mgemm_glu(x.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K, 0, stream()), "dgemm_glu");
     return out;
   }
-  CHECK_RC(docqa_dgemm_glu(x.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K, stream()), "dgemm_glu");
+  const at::Tensor xa = aligned16(x);
+  CHECK_RC(docqa_dgemm_glu(xa.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K, stream()), "dgemm_glu");
   return out;
 }
 
@@ -761,7 +762,8 @@ at::Tensor dgemm_partial(const at::Tensor& x, const at::Tensor& w, int64_t split
                          stream()), "dgemm_partial");
     return part;
   }
-  CHECK_RC(docqa_dgemm_partial(x.data_ptr(), w.data_ptr(), part.data_ptr<float>(), M, N, K, (int)splits,
+  const at::Tensor xa = aligned16(x);
+  CHECK_RC(docqa_dgemm_partial(xa.data_ptr(), w.data_ptr(), part.data_ptr<float>(), M, N, K, (int)splits,
                                (int)tile_rows, stream()), "dgemm_partial");
   return part;
 }
@@ -869,7 +871,8 @@ at::Tensor dgemm(const at::Tensor& x, const at::Tensor& w, int64_t splits) {
   }
   at::Tensor part;
   if (S > 1) part = at::empty({S, M, N}, x.options().dtype(at::kFloat));
-  CHECK_RC(docqa_dgemm(x.data_ptr(), w.data_ptr(), out.data_ptr(), S > 1 ? part.data_ptr<float>() : nullptr,
+  const at::Tensor xa = aligned16(x);
+  CHECK_RC(docqa_dgemm(xa.data_ptr(), w.data_ptr(), out.data_ptr(), S > 1 ? part.data_ptr<float>() : nullptr,
                        M, N, K, S, stream()), "dgemm");
   return out;
 }
@@ -1005,7 +1008,8 @@ std::tuple<at::Tensor, at::Tensor> dgemm_argmax_val(const at::Tensor& x, const a
   auto outv = at::empty({M}, x.options().dtype(at::kFloat));
   auto ws_v = at::empty({M, N / 64}, x.options().dtype(at::kFloat));
   auto ws_i = at::empty({M, N / 64}, x.options().dtype(at::kInt));
-  CHECK_RC(docqa_dgemm_argmax(x.data_ptr(), w.data_ptr(), out.data_ptr<int64_t>(), outv.data_ptr<float>(),
+  const at::Tensor xa = aligned16(x);
+  CHECK_RC(docqa_dgemm_argmax(xa.data_ptr(), w.data_ptr(), out.data_ptr<int64_t>(), outv.data_ptr<float>(),
                               ws_v.data_ptr<float>(), ws_i.data_ptr<int>(), M, N, K, (int)n_valid, stream()),
            "dgemm_argmax");
   return {out, outv};

@@ -45,4 +45,10 @@ static void debug_sync(const char* name) {
     if (kernel_debug()) debug_sync(name);                                                  \
   } while (0)
 
+// x, or a copy of it where its storage offset is not a multiple of 16 bytes: rows that go straight into
+// LDS are read in 16-byte pieces
+inline at::Tensor aligned16(const at::Tensor& x) {
+  return (reinterpret_cast<uintptr_t>(x.data_ptr()) & 15u) == 0 ? x : x.clone();
+}
+
 }  // namespace

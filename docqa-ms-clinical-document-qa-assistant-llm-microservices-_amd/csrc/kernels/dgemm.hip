@@ -23,11 +23,10 @@
 //     and no separate silu_mul launch.  7 n-tiles per workgroup (112 rows) make the Llama-3-8B
 //     shape exactly 256 workgroups = one per CU, and halve the L2 traffic of re-reading X
 //     per workgroup (at M = 64 that X traffic, not HBM, was the limiter).
-//   * 65..128 rows: each wave owns two 16-row m-tiles over the whole k-block, so every
-//     B fragment read from the LDS ring feeds two MFMAs and the weights still stream from
-//     HBM exactly once (a second pass over 64-row halves would read them twice).
-// Shapes: N % (16 NT) == 0, (K / S) % 512 == 0 (whole 4-stage ring turns), M <= 128
-// (M <= 192 with 64-row weight tiles: three m-tiles per wave, no fused SwiGLU).
+// That kernel (dgemm_kernel) serves up to 16 rows, where its sums are also the fused-norm forms' bit for
+// bit, and 129..192 rows (64-row weight tiles, three m-tiles per wave, no fused SwiGLU); 17..128 rows take
+// dstream_kernel below, whose X rows come through the LDS ring as well.
+// Shapes: N % (16 NT) == 0, (K / S) % 512 == 0 (whole 4-stage ring turns).
 #include "docqa_common.h"
 #include "docqa_asm.h"
 #include "docqa_argmax.h"
@@ -201,7 +200,7 @@ __device__ __forceinline__ void xnorm_prologue(const XNormIn& xn, int K, int kbe
   __syncthreads();
 }
 
-template <int EPI, int MT, int NT, int NSR, int XA = 2, bool NORM = false, bool XN = false>
+template <int EPI, int MT, int NT, int NSR, bool NORM = false, bool XN = false>
 __global__ __launch_bounds__(256) void dgemm_kernel(const uint16_t* __restrict__ X,
                                                     const uint16_t* __restrict__ W,
                                                     uint16_t* __restrict__ Y,
@@ -210,7 +209,7 @@ __global__ __launch_bounds__(256) void dgemm_kernel(const uint16_t* __restrict__
                                                     int* __restrict__ pi = nullptr, int n_valid = 0,
                                                     NormArgs na = NormArgs{}, XNormIn xn = XNormIn{}) {
   static_assert(!NORM || EPI == EPI_PARTIAL, "the fused norm consumes split-K slabs");
-  static_assert(!XN || (MT == 1 && XA == 2), "the in-LDS input row is the one-row (batch-1) case");
+  static_assert(!XN || MT == 1, "the in-LDS input row is the one-row (batch-1) case");
   constexpr int MPW = MT > 4 ? MT / 4 : 1;       // m-tiles per wave
   constexpr int MTW = MT > 4 ? 4 : MT;           // wave groups along m
   constexpr int KW = 4 / MTW, SPW = KSTEPS / KW;
@@ -314,51 +313,32 @@ __global__ __launch_bounds__(256) void dgemm_kernel(const uint16_t* __restrict__
 #define RING_STEP(I, XC, XN, NW)                                                        \
   wait_vm_n<NW>(XC);                                                                    \
   ring_barrier();                                                                       \
-  load_x(XN, (I) + XA);                                                                 \
+  load_x(XN, (I) + 2);                                                                 \
   stage_w((I) + NSR - 1);                                                               \
   mma(XC, I);
-  if constexpr (XA == 2) {
-    if constexpr (XN) {
-      // weight stages first, then the input row (its loads overlap theirs; waiting for them
-      // retires the stages too -- vmcnt is in order), then the first two X fragments
+  if constexpr (XN) {
+    // weight stages first, then the input row (its loads overlap theirs; waiting for them
+    // retires the stages too -- vmcnt is in order), then the first two X fragments
 #pragma unroll
-      for (int j = 0; j <= NSR - 2; ++j) stage_w(j);
-      xnorm_prologue(xn, K, kbeg, Ks, blockIdx.x == 0 && blockIdx.y == 0, sx, xred);
-      load_x(x0, 0);
-      load_x(x1, 1);
-    } else {
-#pragma unroll
-      for (int j = 0; j <= NSR - 4; ++j) stage_w(j);
-      load_x(x0, 0);
-      stage_w(NSR - 3);
-      load_x(x1, 1);
-      stage_w(NSR - 2);
-    }
-    // nkb % 4 == 0: a break-free 4-step body keeps each X buffer in one register set (an
-    // early exit makes hipcc merge buffers with register copies that read in-flight data)
-    for (int i = 0; i < nkb; i += 4) {
-      RING_STEP(i, x0, x2, VW)
-      RING_STEP(i + 1, x1, x3, VW)
-      RING_STEP(i + 2, x2, x0, VW)
-      RING_STEP(i + 3, x3, x1, VW)
-    }
-  } else {
-    // X three k-blocks ahead (the 65-128-row case, where X -- not W -- is the longer
-    // pole): issue W0 X0 W1 X1 W2 X2 | step i: X(i+3) W(i+3).  W(i) now follows X(i), and
-    // the ops after W(i) are X(i+1) W(i+1) X(i+2) W(i+2): vmcnt(2 (NT + XR)) retires both.
-    static_assert(NSR == 4, "X-ahead-3 schedule is written for a 4-slot ring");
-    stage_w(0);
+    for (int j = 0; j <= NSR - 2; ++j) stage_w(j);
+    xnorm_prologue(xn, K, kbeg, Ks, blockIdx.x == 0 && blockIdx.y == 0, sx, xred);
     load_x(x0, 0);
-    stage_w(1);
     load_x(x1, 1);
-    stage_w(2);
-    load_x(x2, 2);
-    for (int i = 0; i < nkb; i += 4) {
-      RING_STEP(i, x0, x3, 2 * (NT + XR))
-      RING_STEP(i + 1, x1, x0, 2 * (NT + XR))
-      RING_STEP(i + 2, x2, x1, 2 * (NT + XR))
-      RING_STEP(i + 3, x3, x2, 2 * (NT + XR))
-    }
+  } else {
+#pragma unroll
+    for (int j = 0; j <= NSR - 4; ++j) stage_w(j);
+    load_x(x0, 0);
+    stage_w(NSR - 3);
+    load_x(x1, 1);
+    stage_w(NSR - 2);
+  }
+  // nkb % 4 == 0: a break-free 4-step body keeps each X buffer in one register set (an
+  // early exit makes hipcc merge buffers with register copies that read in-flight data)
+  for (int i = 0; i < nkb; i += 4) {
+    RING_STEP(i, x0, x2, VW)
+    RING_STEP(i + 1, x1, x3, VW)
+    RING_STEP(i + 2, x2, x0, VW)
+    RING_STEP(i + 3, x3, x1, VW)
   }
 #undef RING_STEP
   // drain the clamped tail loads; naming every X buffer keeps their registers reserved
@@ -500,6 +480,216 @@ __global__ __launch_bounds__(256) void dgemm_kernel(const uint16_t* __restrict__
   }
 }
 
+// ---------------------------------------------------------------------------------------
+// 17..128 rows: X and W tiles through one LDS ring, TM X rows x TN weight rows x one K slice a workgroup.
+// Such a product is bound by what a CU can fetch: its weights once from HBM and X again for every TN
+// weight rows from L2, so both arrive as whole 128-byte lines straight into LDS (as MFMA fragments read
+// into registers, 64 bytes a row, X cost as much as W: 128 rows of 28672 x 4096 59 us, so 52; of
+// 4096 x 14336 39.5 -> 31.5, 4096 x 4096 16.3 -> 12.2, 32000 x 4096 87.6 -> 61; 32 rows of the last
+// 53.6 -> 48).  Stages are 64 k's deep, NSR of them, OCC workgroups a CU.  WM x WN waves share the tile;
+// with one tile a workgroup the 4 waves take a 16-deep k-step each instead, so every fragment is read
+// from LDS once, and their sums meet in LDS.
+template <int EPI, int TM, int TN, int WM, int WN, int NSR, int OCC>
+__global__ __launch_bounds__(256, OCC) void dstream_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ W,
+                                                           uint16_t* __restrict__ Y, float* __restrict__ P, int M, int N,
+                                                           int K, int Ks, int xcd_remap, float* __restrict__ pv,
+                                                           int* __restrict__ pi, int n_valid) {
+  constexpr int WK = 4 / (WM * WN);                     // waves along k
+  static_assert(WK == 1 || WK == 4, "all waves on the tile, or all along k");
+  constexpr int ROWB = 128, XST = TM * ROWB, STAGE = XST + TN * ROWB;
+  constexpr int LX = TM / 32, LW = TN / 32, L = LX + LW;   // 16-B loads a thread and stage
+  constexpr int TI = TM / WM / 32, TJ = TN / WN / 32, KS = 4 / WK;
+  __shared__ __attribute__((aligned(16))) char smem[NSR * STAGE];
+  static_assert(WK == 1 || 4 * TI * TJ * 4096 <= NSR * STAGE, "the waves' sums");
+  static_assert(EPI != EPI_ARGMAX || TM * (TN + 1) * 4 <= NSR * STAGE, "the logits tile");
+  int tile = blockIdx.x, slice = blockIdx.y;
+  if (xcd_remap) {   // as in dgemm_kernel: an XCD runs one slice, whose X stays in its L2
+    const int S = gridDim.y, wg = blockIdx.x + blockIdx.y * gridDim.x, xcd = wg & 7;
+    slice = xcd % S;
+    tile = (wg >> 3) * (8 / S) + xcd / S;
+  }
+  const int n0 = tile * TN, kbeg = slice * Ks;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hh = lane >> 5;
+  const int wk = wave % WK, wm = wave / WK % WM, wn = wave / WK / WM;
+  const uint32_t ring = lds_u32(smem);
+  auto swz = [](int row, int ch) { return ch ^ ((row >> 1) & 7); };   // 32-row fragment reads hit distinct banks
+
+  const char* xb = (const char*)(X + kbeg);
+  const char* wb = (const char*)(W + (size_t)n0 * K + kbeg);
+  uint32_t offx[LX], offw[LW];
+#pragma unroll
+  for (int i = 0; i < LX; ++i) {
+    const int r = i * 32 + (tid >> 3);
+    offx[i] = (uint32_t)min(r, M - 1) * (uint32_t)(K * 2) + swz(r, tid & 7) * 16;
+  }
+#pragma unroll
+  for (int i = 0; i < LW; ++i) {
+    const int r = i * 32 + (tid >> 3);
+    offw[i] = (uint32_t)r * (uint32_t)(K * 2) + swz(r, tid & 7) * 16;
+  }
+  // past the last stage the sources are clamped, so that every step issues the same loads
+  const int nk = Ks / 64;
+  auto stage = [&](int kt, int buf) {
+    const uint32_t d = ring + (uint32_t)(buf * STAGE + wave * 1024), k = (uint32_t)min(kt, nk - 1) * ROWB;
+#pragma unroll
+    for (int i = 0; i < LW; ++i) glds16<true>(wb + (size_t)(offw[i] + k), __builtin_amdgcn_readfirstlane(d + XST + i * 4096));
+#pragma unroll
+    for (int i = 0; i < LX; ++i) glds16_off(xb, offx[i] + k, __builtin_amdgcn_readfirstlane(d + i * 4096));
+  };
+
+  f32x16 acc[TJ][TI];
+#pragma unroll
+  for (int n = 0; n < TJ; ++n)
+#pragma unroll
+    for (int m = 0; m < TI; ++m)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[n][m][r] = 0.f;
+#pragma unroll
+  for (int t = 0; t < NSR - 1; ++t) stage(t, t);
+  int buf = 0;
+  for (int kt = 0; kt < nk; ++kt) {
+    wait_vmcnt<(NSR - 2) * L>();                        // stage kt has landed
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    ring_barrier();                                     // for every wave, and all have read what is overwritten next
+    stage(kt + NSR - 1, buf ? buf - 1 : NSR - 1);
+    const char* sx = smem + buf * STAGE;
+    const char* sw = sx + XST;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int ch = (wk * KS + ks) * 2 + hh;
+      bf16x8 a[TI], w[TJ];
+#pragma unroll
+      for (int i = 0; i < TJ; ++i) {
+        const int r = (wn * TJ + i) * 32 + l32;
+        w[i] = *reinterpret_cast<const bf16x8*>(sw + r * ROWB + swz(r, ch) * 16);
+      }
+#pragma unroll
+      for (int i = 0; i < TI; ++i) {
+        const int r = (wm * TI + i) * 32 + l32;
+        a[i] = *reinterpret_cast<const bf16x8*>(sx + r * ROWB + swz(r, ch) * 16);
+      }
+#pragma unroll
+      for (int n = 0; n < TJ; ++n)
+#pragma unroll
+        for (int m = 0; m < TI; ++m) acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[n], a[m], acc[n][m], 0, 0, 0);
+    }
+    buf = buf == NSR - 1 ? 0 : buf + 1;
+  }
+  wait_vmcnt<0>();                                      // the clamped tail has landed too
+  __syncthreads();
+
+  // Four consecutive weight rows 8 g + 4 hh of a 32 x 32 tile, at X row l32, are one register quad.  A wave
+  // along k takes quad g = wk of every tile's sum.
+  constexpr int GQ = WK == 1 ? 4 : 1;
+  float* part = reinterpret_cast<float*>(smem);
+  auto slot = [&](int w, int n, int m, int g) { return part + ((((w * TJ + n) * TI + m) * 4 + g) * 64 + lane) * 4; };
+  auto own = [&](int n, int m, int g) {
+    return f32x4{acc[n][m][4 * g], acc[n][m][4 * g + 1], acc[n][m][4 * g + 2], acc[n][m][4 * g + 3]};
+  };
+  if constexpr (WK > 1) {
+#pragma unroll
+    for (int n = 0; n < TJ; ++n)
+#pragma unroll
+      for (int m = 0; m < TI; ++m)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) *reinterpret_cast<f32x4*>(slot(wave, n, m, g)) = own(n, m, g);
+    __syncthreads();
+  }
+  auto quad = [&](int n, int m, int g) {
+    if constexpr (WK == 1) {
+      return own(n, m, g);
+    } else {
+      f32x4 v = *reinterpret_cast<const f32x4*>(slot(0, n, m, g));
+#pragma unroll
+      for (int w = 1; w < WK; ++w) v += *reinterpret_cast<const f32x4*>(slot(w, n, m, g));
+      return v;
+    }
+  };
+  auto x_row = [&](int m) { return (wm * TI + m) * 32 + l32; };
+  auto w_col = [&](int n, int g) { return (wn * TJ + n) * 32 + 8 * g + 4 * hh; };
+
+  if constexpr (EPI == EPI_ARGMAX) {
+    // the logits tile through LDS, 4 lanes a row -> one (value, id) partial per (row, tile)
+    f32x4 v[TJ][TI][GQ];
+#pragma unroll
+    for (int n = 0; n < TJ; ++n)
+#pragma unroll
+      for (int m = 0; m < TI; ++m)
+#pragma unroll
+        for (int q = 0; q < GQ; ++q) v[n][m][q] = quad(n, m, WK == 1 ? q : wk);
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < TJ; ++n)
+#pragma unroll
+      for (int m = 0; m < TI; ++m)
+#pragma unroll
+        for (int q = 0; q < GQ; ++q)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            part[x_row(m) * (TN + 1) + w_col(n, WK == 1 ? q : wk) + e] = v[n][m][q][e];
+    __syncthreads();
+    const int parts = N / BN;                           // of 64 columns, as many as the workspace's row has
+    for (int i = tid >> 2; i < TM * (TN / BN); i += 64) {
+      const int rr = i % TM, half = i / TM, c0 = half * BN + (tid & 3) * (BN / 4);
+      float bv = -FLT_MAX;
+      int bi = 0x7fffffff;
+#pragma unroll 4
+      for (int c = c0; c < c0 + BN / 4; ++c)
+        if (n0 + c < n_valid) argmax_better(bv, bi, bf2f(f2bf(part[rr * (TN + 1) + c])), n0 + c);
+#pragma unroll
+      for (int o = 1; o <= 2; o <<= 1) {
+        const float ov = __shfl_xor(bv, o, 64);
+        const int oi = __shfl_xor(bi, o, 64);
+        argmax_better(bv, bi, ov, oi);
+      }
+      if ((tid & 3) == 0 && rr < M) {
+        pv[(size_t)rr * parts + tile * (TN / BN) + half] = bv;
+        pi[(size_t)rr * parts + tile * (TN / BN) + half] = bi;
+      }
+    }
+  } else if constexpr (EPI == EPI_GLU) {
+    // quads g and g + 1 are 4 gate rows and their up rows; the sums as the unfused product's bf16
+    if (WK > 1 && wk >= 2) return;
+#pragma unroll
+    for (int n = 0; n < TJ; ++n)
+#pragma unroll
+      for (int m = 0; m < TI; ++m)
+#pragma unroll
+        for (int q = 0; q < (WK == 1 ? 2 : 1); ++q) {
+          const int g = 2 * (WK == 1 ? q : wk), row = x_row(m);
+          const f32x4 v = quad(n, m, g), u = quad(n, m, g + 1);
+          float o[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] = silu_f(bf2f(f2bf(v[e]))) * bf2f(f2bf(u[e]));
+          if (row < M)
+            *reinterpret_cast<uint2*>(Y + (size_t)row * (N >> 1) + ((n0 + (wn * TJ + n) * 32 + 8 * g) >> 1) + 4 * hh) =
+                make_uint2(pack2(o[0], o[1]), pack2(o[2], o[3]));
+        }
+  } else {
+#pragma unroll
+    for (int n = 0; n < TJ; ++n)
+#pragma unroll
+      for (int m = 0; m < TI; ++m)
+#pragma unroll
+        for (int q = 0; q < GQ; ++q) {
+          const int g = WK == 1 ? q : wk, row = x_row(m);
+          const f32x4 v = quad(n, m, g);
+          if (row >= M) continue;
+          if constexpr (EPI == EPI_PARTIAL) {
+            *reinterpret_cast<f32x4*>(P + ((size_t)slice * M + row) * N + n0 + w_col(n, g)) = v;
+          } else {
+            float o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              o[e] = EPI == EPI_RELU2 ? relu2(v[e]) : EPI == EPI_GELU ? gelu_tanh(v[e]) : v[e];
+            *reinterpret_cast<uint2*>(Y + (size_t)row * N + n0 + w_col(n, g)) =
+                make_uint2(pack2(o[0], o[1]), pack2(o[2], o[3]));
+          }
+        }
+  }
+}
+
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ P,
                                                             uint16_t* __restrict__ Y, int MN, int S) {
   const int i = (blockIdx.x * 256 + threadIdx.x) * 4;
@@ -525,14 +715,6 @@ int docqa_dgemm_splits(int N, int K) {
   return s;
 }
 
-static int xa_knob() {   // X prefetch distance for 65-128 rows (tuning experiments)
-  static const int v = [] {
-    const char* e = getenv("DOCQA_DGEMM_XA");
-    return e ? atoi(e) : 0;
-  }();
-  return v;
-}
-
 static int xcd_knob() {   // XCD-aware slice placement (A/B experiments): 1 on, 0 off
   static const int v = [] {
     const char* e = getenv("DOCQA_DGEMM_XCD");
@@ -541,26 +723,51 @@ static int xcd_knob() {   // XCD-aware slice placement (A/B experiments): 1 on, 
   return v;
 }
 
-template <int EPI, int NT, int NSR = NS>
-static void launch_mt(int mt, dim3 grid, hipStream_t s, const uint16_t* x, const uint16_t* w,
-                      uint16_t* y, float* p, int M, int N, int K, int Ks, float* pv = nullptr,
-                      int* pi = nullptr, int nv = 0) {
+static bool remap_slices(dim3 grid) {
   const int S = grid.y;
-  const int xr = (xcd_knob() && S > 1 && 8 % S == 0 && (grid.x * S) % 8 == 0) ? 1 : 0;
-  if (mt == 1) dgemm_kernel<EPI, 1, NT, NSR><<<grid, 256, 0, s>>>(x, w, y, p, M, N, K, Ks, xr, pv, pi, nv);
-  else if (mt == 2) dgemm_kernel<EPI, 2, NT, NSR><<<grid, 256, 0, s>>>(x, w, y, p, M, N, K, Ks, xr, pv, pi, nv);
-  else if (mt <= 4) dgemm_kernel<EPI, 4, NT, NSR><<<grid, 256, 0, s>>>(x, w, y, p, M, N, K, Ks, xr, pv, pi, nv);
-  else if (mt <= 8) {
-    if constexpr (NSR == 4) {
-      if (xa_knob() == 3)
-        dgemm_kernel<EPI, 8, NT, NSR, 3><<<grid, 256, 0, s>>>(x, w, y, p, M, N, K, Ks, xr, pv, pi, nv);
-      else dgemm_kernel<EPI, 8, NT, NSR><<<grid, 256, 0, s>>>(x, w, y, p, M, N, K, Ks, xr, pv, pi, nv);
+  return xcd_knob() && S > 1 && 8 % S == 0 && (grid.x * S) % 8 == 0;
+}
+
+// the fused SwiGLU on 112-row weight tiles, any m-tile count
+static void launch_glu7(int mt, dim3 grid, hipStream_t s, const uint16_t* x, const uint16_t* w, uint16_t* y, int M,
+                        int N, int K) {
+  if (mt == 1) dgemm_kernel<EPI_GLU, 1, 7, NS><<<grid, 256, 0, s>>>(x, w, y, nullptr, M, N, K, K, 0);
+  else if (mt == 2) dgemm_kernel<EPI_GLU, 2, 7, NS><<<grid, 256, 0, s>>>(x, w, y, nullptr, M, N, K, K, 0);
+  else if (mt <= 4) dgemm_kernel<EPI_GLU, 4, 7, NS><<<grid, 256, 0, s>>>(x, w, y, nullptr, M, N, K, K, 0);
+  else dgemm_kernel<EPI_GLU, 8, 7, NS><<<grid, 256, 0, s>>>(x, w, y, nullptr, M, N, K, K, 0);
+}
+
+// N % 64 == 0.  Up to 16 rows and 129..192: the ring of weights alone.  Between them X goes through the
+// ring too, on the X rows' next power of two x 64 weight rows; us of 64 / 128 weight rows for 128 rows, and
+// of two / three workgroups a CU for 32 rows, by what fills the chip:
+//   128 rows: 500 and 448 workgroups of 64 (N 32000 and 28672 x K 4096) 67.8 / 61.3 and 63.2 / 52.9, 384
+//     (6144 x 4096 S 4) 20.1 / 17.9; 256 of 64 (16384 x 4096) 36.4 / 39.1, (4096 x 4096 S 4) 12.2 / 15;
+//   32 rows: 500 and 448 of them 51.5 / 48.1 and 45.6 / 44.2, 192 (6144 x 4096 S 2) 12.7 / 13.2.
+// (With 8 waves on 128 x 128 tiles, 2 x 4 or two groups along k: 52.7 - 53.8 for 52.9.)
+template <int EPI>
+static void launch_rows(dim3 grid, hipStream_t s, const uint16_t* x, const uint16_t* w, uint16_t* y, float* p, int M,
+                        int N, int K, int Ks, float* pv = nullptr, int* pi = nullptr, int nv = 0) {
+  const int mt = (M + 15) / 16;
+  int xr = remap_slices(grid);
+  if (mt == 1) {
+    dgemm_kernel<EPI, 1, 4, NS><<<grid, 256, 0, s>>>(x, w, y, p, M, N, K, Ks, xr, pv, pi, nv);
+  } else if (mt == 2) {
+    if (grid.x * grid.y > 256)
+      dstream_kernel<EPI, 32, 64, 1, 1, 4, 3><<<grid, 256, 0, s>>>(x, w, y, p, M, N, K, Ks, xr, pv, pi, nv);
+    else
+      dstream_kernel<EPI, 32, 64, 1, 1, 6, 2><<<grid, 256, 0, s>>>(x, w, y, p, M, N, K, Ks, xr, pv, pi, nv);
+  } else if (mt <= 4) {
+    dstream_kernel<EPI, 64, 64, 1, 1, 5, 2><<<grid, 256, 0, s>>>(x, w, y, p, M, N, K, Ks, xr, pv, pi, nv);
+  } else if (mt <= 8) {
+    const dim3 wide(N / 128, grid.y);
+    if (N % 128 == 0 && wide.x * wide.y >= 192) {
+      xr = remap_slices(wide);
+      dstream_kernel<EPI, 128, 128, 2, 2, 5, 1><<<wide, 256, 0, s>>>(x, w, y, p, M, N, K, Ks, xr, pv, pi, nv);
     } else {
-      dgemm_kernel<EPI, 8, NT, NSR><<<grid, 256, 0, s>>>(x, w, y, p, M, N, K, Ks, xr, pv, pi, nv);
+      dstream_kernel<EPI, 128, 64, 2, 2, 3, 2><<<grid, 256, 0, s>>>(x, w, y, p, M, N, K, Ks, xr, pv, pi, nv);
     }
-  } else if constexpr (NT <= 8 && EPI != EPI_GLU) {
-    // 129-192 rows: three m-tiles per wave
-    dgemm_kernel<EPI, 12, NT, NSR><<<grid, 256, 0, s>>>(x, w, y, p, M, N, K, Ks, xr, pv, pi, nv);
+  } else if constexpr (EPI != EPI_GLU) {
+    dgemm_kernel<EPI, 12, 4, NS><<<grid, 256, 0, s>>>(x, w, y, p, M, N, K, Ks, xr, pv, pi, nv);
   }
 }
 
@@ -573,13 +780,12 @@ int docqa_dgemm(const void* X, const void* W, void* Y, float* partial, int M, in
   if (M == 0) return 0;
   if (!shape_ok(M, N, K, S, BN) || (S > 1 && !partial)) return -1;
   dim3 grid(N / BN, S);
-  const int mt = (M + 15) / 16;
   const uint16_t* x = (const uint16_t*)X;
   const uint16_t* w = (const uint16_t*)W;
   if (S == 1) {
-    launch_mt<EPI_BF16, 4>(mt, grid, s, x, w, (uint16_t*)Y, nullptr, M, N, K, K);
+    launch_rows<EPI_BF16>(grid, s, x, w, (uint16_t*)Y, nullptr, M, N, K, K);
   } else {
-    launch_mt<EPI_PARTIAL, 4>(mt, grid, s, x, w, nullptr, partial, M, N, K, K / S);
+    launch_rows<EPI_PARTIAL>(grid, s, x, w, nullptr, partial, M, N, K, K / S);
     const int MN = M * N;  // multiple of 4 (N % 64 == 0)
     splitk_reduce_kernel<<<(MN / 4 + 255) / 256, 256, 0, s>>>(partial, (uint16_t*)Y, MN, S);
   }
@@ -592,11 +798,9 @@ int docqa_dgemm_act(const void* X, const void* W, void* Y, int act, int M, int N
   if (M == 0) return 0;
   if (!shape_ok(M, N, K, 1, BN)) return -1;
   if (act == ACT_RELU2)
-    launch_mt<EPI_RELU2, 4>((M + 15) / 16, dim3(N / BN, 1), s, (const uint16_t*)X, (const uint16_t*)W, (uint16_t*)Y,
-                            nullptr, M, N, K, K);
+    launch_rows<EPI_RELU2>(dim3(N / BN, 1), s, (const uint16_t*)X, (const uint16_t*)W, (uint16_t*)Y, nullptr, M, N, K, K);
   else if (act == ACT_GELU_TANH)
-    launch_mt<EPI_GELU, 4>((M + 15) / 16, dim3(N / BN, 1), s, (const uint16_t*)X, (const uint16_t*)W, (uint16_t*)Y,
-                           nullptr, M, N, K, K);
+    launch_rows<EPI_GELU>(dim3(N / BN, 1), s, (const uint16_t*)X, (const uint16_t*)W, (uint16_t*)Y, nullptr, M, N, K, K);
   else
     return -1;
   DOCQA_CHECK_LAUNCH();
@@ -609,21 +813,7 @@ int docqa_dgemm_partial(const void* X, const void* W, float* P, int M, int N, in
                         int tile_rows, hipStream_t s) {
   if (M == 0) return 0;
   if (!P || (tile_rows != 64 && tile_rows != 128) || !shape_ok(M, N, K, S, tile_rows)) return -1;
-  const int mt = (M + 15) / 16;
-  const uint16_t* x = (const uint16_t*)X;
-  const uint16_t* w = (const uint16_t*)W;
-  static const int ns_env = [] {   // ring depth knob (tuning experiments)
-    const char* e = getenv("DOCQA_DGEMM_NS");
-    return e ? atoi(e) : 0;
-  }();
-  if (tile_rows == 128)   // 1 workgroup per CU (128 KB ring), X re-read half as often
-    launch_mt<EPI_PARTIAL, 8>(mt, dim3(N / 128, S), s, x, w, nullptr, P, M, N, K, K / S);
-  else if (ns_env == 6)
-    launch_mt<EPI_PARTIAL, 4, 6>(mt, dim3(N / 64, S), s, x, w, nullptr, P, M, N, K, K / S);
-  else if (ns_env == 8)
-    launch_mt<EPI_PARTIAL, 4, 8>(mt, dim3(N / 64, S), s, x, w, nullptr, P, M, N, K, K / S);
-  else
-    launch_mt<EPI_PARTIAL, 4>(mt, dim3(N / 64, S), s, x, w, nullptr, P, M, N, K, K / S);
+  launch_rows<EPI_PARTIAL>(dim3(N / BN, S), s, (const uint16_t*)X, (const uint16_t*)W, nullptr, P, M, N, K, K / S);
   DOCQA_CHECK_LAUNCH();
   return 0;
 }
@@ -639,7 +829,7 @@ int docqa_dgemm_add_rmsnorm(const void* X, const void* W, float* P, int M, int N
   NormArgs na{tick, (uint16_t*)residual, (const uint16_t*)gamma, (uint16_t*)out, eps};
   const dim3 grid(N / BN, S);
   const int xr = (xcd_knob() && S > 1 && 8 % S == 0 && (grid.x * S) % 8 == 0) ? 1 : 0;
-  dgemm_kernel<EPI_PARTIAL, 1, 4, NS, 2, true><<<grid, 256, 0, s>>>((const uint16_t*)X, (const uint16_t*)W, nullptr,
+  dgemm_kernel<EPI_PARTIAL, 1, 4, NS, true><<<grid, 256, 0, s>>>((const uint16_t*)X, (const uint16_t*)W, nullptr,
                                                                     P, M, N, K, K / S, xr, nullptr, nullptr, 0, na);
   DOCQA_CHECK_LAUNCH();
   return 0;
@@ -661,7 +851,7 @@ int docqa_dgemm_partial_xn(const float* Pin, int Sin, const void* res_in, void* 
   const int xr = (xcd_knob() && S > 1 && 8 % S == 0 && (grid.x * S) % 8 == 0) ? 1 : 0;
   // (an 8-slot ring to stream on under the input-row prologue measured slower: QKV 17.7 vs
   // 16.4 us, profiles/r4_b1_ab.log)
-  dgemm_kernel<EPI_PARTIAL, 1, 4, NS, 2, false, true><<<grid, 256, 0, s>>>(
+  dgemm_kernel<EPI_PARTIAL, 1, 4, NS, false, true><<<grid, 256, 0, s>>>(
       nullptr, (const uint16_t*)W, nullptr, P, 1, N, K, K / S, xr, nullptr, nullptr, 0, NormArgs{}, xn);
   DOCQA_CHECK_LAUNCH();
   return 0;
@@ -671,10 +861,10 @@ int docqa_dgemm_glu_xn(const float* Pin, int Sin, const void* res_in, void* res_
                        const void* W, void* Y, int N, int K, hipStream_t s) {
   const XNormIn xn{Pin, Sin, (const uint16_t*)res_in, (uint16_t*)res_out, (const uint16_t*)gamma, eps};
   if (xn_ok(N, K, 1, 112, xn) && N / 112 >= 192)
-    dgemm_kernel<EPI_GLU, 1, 7, NS, 2, false, true><<<dim3(N / 112), 256, 0, s>>>(
+    dgemm_kernel<EPI_GLU, 1, 7, NS, false, true><<<dim3(N / 112), 256, 0, s>>>(
         nullptr, (const uint16_t*)W, (uint16_t*)Y, nullptr, 1, N, K, K, 0, nullptr, nullptr, 0, NormArgs{}, xn);
   else if (xn_ok(N, K, 1, 64, xn))
-    dgemm_kernel<EPI_GLU, 1, 4, NS, 2, false, true><<<dim3(N / 64), 256, 0, s>>>(
+    dgemm_kernel<EPI_GLU, 1, 4, NS, false, true><<<dim3(N / 64), 256, 0, s>>>(
         nullptr, (const uint16_t*)W, (uint16_t*)Y, nullptr, 1, N, K, K, 0, nullptr, nullptr, 0, NormArgs{}, xn);
   else
     return -1;
@@ -686,20 +876,18 @@ int docqa_dgemm_glu_xn(const float* Pin, int Sin, const void* res_in, void* res_
 int docqa_dgemm_glu(const void* X, const void* W, void* Y, int M, int N, int K, hipStream_t s) {
   if (M == 0) return 0;
   if (M > 128) return -1;
-  const int mt = (M + 15) / 16;
   const uint16_t* x = (const uint16_t*)X;
   const uint16_t* w = (const uint16_t*)W;
-  static const int glu_nt = [] {   // tile-width knob (tuning experiments): 4 -> 64-row tiles
-    const char* e = getenv("DOCQA_GLU_NT");
-    return e ? atoi(e) : 0;
-  }();
-  if (glu_nt != 4 && shape_ok(M, N, K, 1, 112) && N / 112 >= 192) {
-    launch_mt<EPI_GLU, 7>(mt, dim3(N / 112), s, x, w, (uint16_t*)Y, nullptr, M, N, K, K);
-  } else if (shape_ok(M, N, K, 1, 64)) {
-    launch_mt<EPI_GLU, 4>(mt, dim3(N / 64), s, x, w, (uint16_t*)Y, nullptr, M, N, K, K);
-  } else {
+  // 112-row tiles of the weight ring up to 16 rows and at 33..64 (28672 x 4096, 64 rows: 47.4 us, 64 x 64
+  // tiles 52.2, 64 x 128 of two k-groups 47.3; 32 rows 45.6 - 47.2 against 44.2) and where N has no 64-row tiles
+  const bool wide = shape_ok(M, N, K, 1, 112) && N / 112 >= 192, even = shape_ok(M, N, K, 1, BN);
+  const int mt = (M + 15) / 16;
+  if (wide && (!even || mt == 1 || mt == 3 || mt == 4))
+    launch_glu7(mt, dim3(N / 112), s, x, w, (uint16_t*)Y, M, N, K);
+  else if (even)
+    launch_rows<EPI_GLU>(dim3(N / BN), s, x, w, (uint16_t*)Y, nullptr, M, N, K, K);
+  else
     return -1;
-  }
   DOCQA_CHECK_LAUNCH();
   return 0;
 }
@@ -711,9 +899,8 @@ int docqa_dgemm_argmax(const void* X, const void* W, int64_t* out, float* outv, 
                        int N, int K, int n_valid, hipStream_t s) {
   if (M == 0) return 0;
   if (!shape_ok(M, N, K, 1, BN) || n_valid <= 0 || n_valid > N) return -1;
-  const int mt = (M + 15) / 16;
-  launch_mt<EPI_ARGMAX, 4>(mt, dim3(N / BN), s, (const uint16_t*)X, (const uint16_t*)W, nullptr, nullptr, M, N, K,
-                           K, ws_v, ws_i, n_valid);
+  launch_rows<EPI_ARGMAX>(dim3(N / BN), s, (const uint16_t*)X, (const uint16_t*)W, nullptr, nullptr, M, N, K, K, ws_v,
+                          ws_i, n_valid);
   argmax_merge_kernel<<<M, 256, 0, s>>>(ws_v, ws_i, N / BN, out, outv);
   DOCQA_CHECK_LAUNCH();
   return 0;

@@ -136,7 +136,7 @@ def glu_linear(x, w_il):
     skinny fused-SwiGLU decode GEMM (dgemm.hip); 129..512 rows take the mid-M kernel
     (:func:`mid_plan`), so no decode bucket runs the library GEMM.  Measured vs hipBLASLt +
     silu_mul at M = 64 / 96 / 128: 50.9 / 60.0 / 63.1 us vs 56.4 / 57.6 / 59.7
-    (profiles/r4_lm_head_probe.log)."""
+    (profiles/r4_lm_head_probe.log); with X through the LDS ring 50.5 / 52.3 at 96 / 128."""
     if _gpu(x):
         N, K = w_il.shape
         if x.numel() // K <= 128 and N % 64 == 0 and K % 512 == 0:
@@ -187,7 +187,9 @@ def decode_plan(M: int, N: int, K: int) -> tuple[int, int]:
     LM head and, above 32 rows, gate|up stay on hipBLASLt; at <= 64 rows QKV / O / down use
     64-row tiles with the smallest split giving >= 192 workgroups; at 65-128 rows 128-row
     tiles (X re-read from L2 half as often) where such a split exists (QKV S=4: 21.9 us vs
-    hipBLASLt 25.2 at M=128; O S=8: 17.2 vs 24.4), else 64-row tiles (down S=4: 40.7 vs 75.1)."""
+    hipBLASLt 25.2 at M=128; O S=8: 17.2 vs 24.4), else 64-row tiles (down S=4: 40.7 vs 75.1).
+    With X through the LDS ring (17..128 rows, the width then chosen at the launch) the same plans
+    take QKV 17.9, O at S=4 12.2 and down 31.8 us at M=128; QKV 14.9, O 9.5 and down 23.9 at M=64."""
     if M > 192 or N % 64 or N >= 65536 or (N >= 16384 and M > 32):
         return 0, 64
     if M > 128:
