@@ -2,6 +2,8 @@
 //   C[M, N] = A[M, K] . W[N, K]^T           (bf16 in, fp32 accumulate, bf16 out)
 //   C[M, N/2] = silu(gate) * up             (EPI_GLU: W = the 8-interleaved gate|up rows)
 //   C[M, N] = act(A . W^T)                  (EPI_RELU2, EPI_GELU)
+// Tiles are 256 rows high as described here, or 224, 192 or 160 (pgemm_height): the second m-half of each
+// wave row is then 48, 32 or 16 rows instead of 64, and HA1 and the last two phases shrink with it.
 // Replaces hipBLASLt for the prefill QKV / O / gate|up (+ fused SwiGLU) / down projections
 // (llm-qa/main.py:117 -> prefill inside Ollama in the reference).
 //
@@ -42,7 +44,7 @@
 using namespace docqa;
 
 namespace {
-constexpr int BM = 256, BN = 256, BK = 64;
+constexpr int BN = 256, BK = 64;
 constexpr int HALF_B = 128 * BK * 2;     // bytes of one half-tile (16 KiB)
 constexpr int BUF_B = 4 * HALF_B;        // bytes of one K-tile buffer (64 KiB)
 constexpr int SCR_PITCH = 72;            // epilogue scratch row pitch (bf16), 144 B
@@ -87,12 +89,19 @@ __device__ __forceinline__ void glds_pair(const void* sbase, uint32_t v0, uint32
 
 __device__ __forceinline__ float silu_f(float x) { return x / (1.f + __expf(-x)); }
 
-// K range [kbeg, kbeg + 128 nit) of the 256 x 256 output tile at (m0, n0) into acc (zeroed
+// Output tiles are 32 (4 + MI) rows high: each wave row owns 64 rows and 16 MI (1..4) more, the m-halves.
+template <int MI> constexpr int kTileM = 128 + 32 * MI;
+
+// K range [kbeg, kbeg + 128 nit) of the kTileM<MI> x 256 output tile at (m0, n0) into acc (zeroed
 // here), nit >= 1.  Returns with the wave rows re-aligned and every LDS buffer drained, so
 // the caller may reuse the LDS as epilogue scratch.
+template <int MI>
 __device__ __forceinline__ void pgemm_mainloop(char* smem, const uint16_t* __restrict__ A,
                                                const uint16_t* __restrict__ W, int M, int K, int m0, int n0,
                                                int kbeg, int nit, f32x4 (&acc)[2][4][2][2]) {
+  constexpr int HL = MI > 2 ? 2 : 1;       // wave-instructions a wave issues for HA1 (32 MI rows: 4 MI in all;
+                                           // the ones left over load some of them again, to the same place)
+  constexpr int F = 6 + HL;                // ... for 4 half-tiles
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wr = wave >> 2, wc = wave & 3;
@@ -105,12 +114,14 @@ __device__ __forceinline__ void pgemm_mainloop(char* smem, const uint16_t* __res
   for (int h = 0; h < 4; ++h)
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      const int p = (i * 8 + wave) * 64 + lane;      // physical 16-B chunk of the half-tile
+      const int p = (h == HA1 ? (i * 8 + wave) % (4 * MI) : i * 8 + wave) * 64 + lane;   // physical 16-B chunk
       const int lr = p >> 3;                         // half-tile row 0..127
       const int lc = (p & 7) ^ ((lr >> 1) & 7);      // logical chunk stored there
       int grow;
-      if (h == HA0 || h == HA1) {
-        grow = min(m0 + (lr >> 6) * 128 + (h == HA1 ? 64 : 0) + (lr & 63), M - 1);
+      if (h == HA0) {
+        grow = min(m0 + (lr >> 6) * (kTileM<MI> / 2) + (lr & 63), M - 1);
+      } else if (h == HA1) {
+        grow = min(m0 + lr / (16 * MI) * (kTileM<MI> / 2) + 64 + lr % (16 * MI), M - 1);
       } else {
         grow = n0 + (lr >> 5) * 64 + (h == HB1 ? 32 : 0) + (lr & 31);
       }
@@ -119,8 +130,13 @@ __device__ __forceinline__ void pgemm_mainloop(char* smem, const uint16_t* __res
   // stage half-tile h of K-tile kt into buffer kt & 1
   auto stage = [&](int h, int kt) {
     const uint16_t* base = (h == HA0 || h == HA1 ? A : W) + kbeg + kt * BK;
-    const uint32_t d = __builtin_amdgcn_readfirstlane(lds + (uint32_t)((kt & 1) * BUF_B + h * HALF_B + wave * 1024));
-    glds_pair(base, soff[h][0], soff[h][1], d, d + 8 * 1024);
+    const uint32_t d0 = lds + (uint32_t)((kt & 1) * BUF_B + h * HALF_B);
+    const uint32_t d = __builtin_amdgcn_readfirstlane(d0 + (h == HA1 ? wave % (4 * MI) : wave) * 1024);
+    if (h == HA1 && HL == 1)
+      glds16_off(base, soff[h][0], d);
+    else
+      glds_pair(base, soff[h][0], soff[h][1], d,
+                h == HA1 ? __builtin_amdgcn_readfirstlane(d0 + (8 + wave) % (4 * MI) * 1024) : d + 8 * 1024);
   };
 
 #pragma unroll
@@ -141,8 +157,8 @@ __device__ __forceinline__ void pgemm_mainloop(char* smem, const uint16_t* __res
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        fa[ks][i] = *reinterpret_cast<const bf16x8*>(h + swz(wr * 64 + i * 16 + fr, ks * 4 + fk));
+      for (int i = 0; i < (mh ? MI : 4); ++i)
+        fa[ks][i] = *reinterpret_cast<const bf16x8*>(h + swz(wr * (mh ? 16 * MI : 64) + i * 16 + fr, ks * 4 + fk));
   };
   auto read_b = [&](int buf, int nh) {
     const char* h = sm + buf * BUF_B + (HB0 + nh) * HALF_B;
@@ -157,7 +173,7 @@ __device__ __forceinline__ void pgemm_mainloop(char* smem, const uint16_t* __res
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < (mh ? MI : 4); ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
           acc[mh][i][nh][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[ks][i], fb[nh][ks][j],
@@ -190,7 +206,8 @@ __device__ __forceinline__ void pgemm_mainloop(char* smem, const uint16_t* __res
   // wait that retires it (E.HA0 / HB0 issued in 3 / 4 -> retired by phase 8 -> read in
   // phase 1 of j+1; E.HB1 5 -> 1 -> 2; E.HA1 6 -> 2 -> 3; O.HA0 / HB0 7 / 8 -> 4 -> 5;
   // O.HB1 1 -> 5 -> 6; O.HA1 2 -> 6 -> 7).  The last iteration issues only phases 1-2 and
-  // retires with the counts that keep the same guarantees (8, 8, 8, 4, 2, 0, 0, 0).
+  // retires with the counts that keep the same guarantees (8, 8, 8, 4, 2, 0, 0, 0).  With HL = 1 for
+  // HA1, which is one of any 4 halves in a row, the 8 is 7 (F), the 4 and 2 are 3 and 1.
   // prologue: everything the steady state assumes was issued in iteration -1
   stage(HA0, 0);
   stage(HB0, 0);
@@ -198,28 +215,28 @@ __device__ __forceinline__ void pgemm_mainloop(char* smem, const uint16_t* __res
   stage(HA1, 0);
   stage(HA0, 1);
   stage(HB0, 1);
-  vmcnt<8>();
+  vmcnt<F>();
   sbarrier();
   if (wr == 1) sbarrier();   // stagger: wave row 1 runs one barrier behind
 
   for (int j = 0; j < nit - 1; ++j) {
     const int kt = 2 * j;
-    PGEMM_PHASE(0, 0, 0, 1, 1, stage(HB1, kt + 1), 8)
-    PGEMM_PHASE(0, 0, 1, 0, 1, stage(HA1, kt + 1), 8)
-    PGEMM_PHASE(0, 1, 1, 1, 0, stage(HA0, kt + 2), 8)
-    PGEMM_PHASE(0, 1, 0, 0, 0, stage(HB0, kt + 2), 8)
-    PGEMM_PHASE(1, 0, 0, 1, 1, stage(HB1, kt + 2), 8)
-    PGEMM_PHASE(1, 0, 1, 0, 1, stage(HA1, kt + 2), 8)
-    PGEMM_PHASE(1, 1, 1, 1, 0, stage(HA0, kt + 3), 8)
-    PGEMM_PHASE(1, 1, 0, 0, 0, stage(HB0, kt + 3), 8)
+    PGEMM_PHASE(0, 0, 0, 1, 1, stage(HB1, kt + 1), F)
+    PGEMM_PHASE(0, 0, 1, 0, 1, stage(HA1, kt + 1), F)
+    PGEMM_PHASE(0, 1, 1, 1, 0, stage(HA0, kt + 2), F)
+    PGEMM_PHASE(0, 1, 0, 0, 0, stage(HB0, kt + 2), F)
+    PGEMM_PHASE(1, 0, 0, 1, 1, stage(HB1, kt + 2), F)
+    PGEMM_PHASE(1, 0, 1, 0, 1, stage(HA1, kt + 2), F)
+    PGEMM_PHASE(1, 1, 1, 1, 0, stage(HA0, kt + 3), F)
+    PGEMM_PHASE(1, 1, 0, 0, 0, stage(HB0, kt + 3), F)
   }
   {
     const int kt = 2 * (nit - 1);
-    PGEMM_PHASE(0, 0, 0, 1, 1, stage(HB1, kt + 1), 8)
-    PGEMM_PHASE(0, 0, 1, 0, 1, stage(HA1, kt + 1), 8)
-    PGEMM_PHASE(0, 1, 1, 1, 0, (void)0, 8)
-    PGEMM_PHASE(0, 1, 0, 0, 0, (void)0, 4)
-    PGEMM_PHASE(1, 0, 0, 1, 1, (void)0, 2)
+    PGEMM_PHASE(0, 0, 0, 1, 1, stage(HB1, kt + 1), F)
+    PGEMM_PHASE(0, 0, 1, 0, 1, stage(HA1, kt + 1), F)
+    PGEMM_PHASE(0, 1, 1, 1, 0, (void)0, F)
+    PGEMM_PHASE(0, 1, 0, 0, 0, (void)0, 2 + HL)
+    PGEMM_PHASE(1, 0, 0, 1, 1, (void)0, HL)
     PGEMM_PHASE(1, 0, 1, 0, 1, (void)0, 0)
     PGEMM_PHASE(1, 1, 1, 1, 0, (void)0, 0)
     PGEMM_PHASE(1, 1, 0, 0, 0, (void)0, 0)
@@ -232,7 +249,7 @@ __device__ __forceinline__ void pgemm_mainloop(char* smem, const uint16_t* __res
 }
 
 // the tile's epilogue through the drained LDS: bf16 tile, fused SwiGLU, or an fp32 slab
-template <int EPI>
+template <int EPI, int MI>
 __device__ __forceinline__ void pgemm_store(char* smem, f32x4 (&acc)[2][4][2][2], uint16_t* __restrict__ C,
                                             float* __restrict__ P, int M, int N, int m0, int n0, int slice) {
   const int tid = threadIdx.x, lane = tid & 63;
@@ -240,13 +257,14 @@ __device__ __forceinline__ void pgemm_store(char* smem, f32x4 (&acc)[2][4][2][2]
   const int wr = wave >> 2, wc = wave & 3;
   const int fr = lane & 15, fk = lane >> 4;
 
-  // ---- epilogue: the wave's 128 x 64 tile -> bf16 scratch [128][SCR_PITCH] -> row stores
+  // ---- epilogue: the wave's WR x 64 tile -> bf16 scratch [WR][SCR_PITCH] -> row stores
+  constexpr int WR = kTileM<MI> / 2;
   uint16_t* scr = reinterpret_cast<uint16_t*>(smem) + wave * 128 * SCR_PITCH;
   if constexpr (EPI == EPI_BF16 || EPI == EPI_RELU2 || EPI == EPI_GELU) {
 #pragma unroll
     for (int mh = 0; mh < 2; ++mh)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < (mh ? MI : 4); ++i)
 #pragma unroll
         for (int nh = 0; nh < 2; ++nh)
 #pragma unroll
@@ -260,9 +278,9 @@ __device__ __forceinline__ void pgemm_store(char* smem, f32x4 (&acc)[2][4][2][2]
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     // 8 lanes per 128-B row segment, 8 rows per sweep
 #pragma unroll 4
-    for (int it = 0; it < 16; ++it) {
+    for (int it = 0; it < WR / 8; ++it) {
       const int r = it * 8 + (lane >> 3), c = (lane & 7) * 8;
-      const int row = m0 + wr * 128 + r;
+      const int row = m0 + wr * WR + r;
       const uint4 v = *reinterpret_cast<const uint4*>(scr + r * SCR_PITCH + c);
       if (row < M) *reinterpret_cast<uint4*>(C + (size_t)row * N + n0 + wc * 64 + c) = v;
     }
@@ -274,7 +292,7 @@ __device__ __forceinline__ void pgemm_store(char* smem, f32x4 (&acc)[2][4][2][2]
 #pragma unroll
     for (int mh = 0; mh < 2; ++mh) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < (mh ? MI : 4); ++i)
 #pragma unroll
         for (int nh = 0; nh < 2; ++nh)
 #pragma unroll
@@ -284,9 +302,9 @@ __device__ __forceinline__ void pgemm_store(char* smem, f32x4 (&acc)[2][4][2][2]
               fs[(i * 16 + fk * 4 + r) * 68 + nh * 32 + j * 16 + fr] = acc[mh][i][nh][j][r];
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll 4
-      for (int it = 0; it < 16; ++it) {
+      for (int it = 0; it < (mh ? 4 * MI : 16); ++it) {
         const int r = it * 4 + (lane >> 4), c = (lane & 15) * 4;
-        const int row = m0 + wr * 128 + mh * 64 + r;
+        const int row = m0 + wr * WR + mh * 64 + r;
         const float4 v = *reinterpret_cast<const float4*>(fs + r * 68 + c);
         if (row < M) *reinterpret_cast<float4*>(Ps + (size_t)row * N + n0 + wc * 64 + c) = v;
       }
@@ -298,7 +316,7 @@ __device__ __forceinline__ void pgemm_store(char* smem, f32x4 (&acc)[2][4][2][2]
 #pragma unroll
     for (int mh = 0; mh < 2; ++mh)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < (mh ? MI : 4); ++i)
 #pragma unroll
         for (int nh = 0; nh < 2; ++nh)
 #pragma unroll
@@ -315,16 +333,16 @@ __device__ __forceinline__ void pgemm_store(char* smem, f32x4 (&acc)[2][4][2][2]
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     // 32 outputs (64 B) per row: 4 lanes per row, 16 rows per sweep
 #pragma unroll 4
-    for (int it = 0; it < 8; ++it) {
+    for (int it = 0; it < WR / 16; ++it) {
       const int r = it * 16 + (lane >> 2), c = (lane & 3) * 8;
-      const int row = m0 + wr * 128 + r;
+      const int row = m0 + wr * WR + r;
       const uint4 v = *reinterpret_cast<const uint4*>(scr + r * SCR_PITCH + c);
       if (row < M) *reinterpret_cast<uint4*>(C + (size_t)row * (N >> 1) + ((n0 + wc * 64) >> 1) + c) = v;
     }
   }
 }
 
-template <int EPI>
+template <int EPI, int MI>
 __global__ __launch_bounds__(512, 2) void pgemm_kernel(const uint16_t* __restrict__ A,
                                                       const uint16_t* __restrict__ W,
                                                       uint16_t* __restrict__ C, float* __restrict__ P,
@@ -355,11 +373,11 @@ __global__ __launch_bounds__(512, 2) void pgemm_kernel(const uint16_t* __restric
   const int gm = min(ntm - first_m, GM);
   const int rem = wg - grp * per_group;
   const int bm = first_m + rem % gm, bn = rem / gm;
-  const int m0 = bm * BM, n0 = bn * BN;
+  const int m0 = bm * kTileM<MI>, n0 = bn * BN;
 
   f32x4 acc[2][4][2][2];
-  pgemm_mainloop(smem, A, W, M, K, m0, n0, kbeg, Ks / (2 * BK), acc);
-  pgemm_store<EPI>(smem, acc, C, P, M, N, m0, n0, slice);
+  pgemm_mainloop<MI>(smem, A, W, M, K, m0, n0, kbeg, Ks / (2 * BK), acc);
+  pgemm_store<EPI, MI>(smem, acc, C, P, M, N, m0, n0, slice);
 }
 }  // namespace
 
@@ -368,6 +386,25 @@ bool docqa_pgemm_ok(int M, int N, int K) {
   // 32-bit per-lane byte offsets: (rows - 1) * K * 2 + 128 must fit
   const uint64_t rows = (uint64_t)(M > N ? M : N);
   return rows * (uint64_t)K * 2ull < (1ull << 32);
+}
+
+// Tile height (as MI) for M rows and `per_row` workgroups a row of tiles: 256 rows are the fastest tile, but
+// a launch takes whole rounds of 256 of them and pads the last row of tiles, so lower ones win where they end
+// sooner.  A round costs 195 + h rows' worth, and the tiles' work as such (the clock falls with it) h / 153
+// each: fitted to 124 launches (8B projections, S 1..4, 530..8200 rows; the choice is 0.3 % off the best of
+// the four on average, 256 rows alone 13 %).  us at 256 / 224 / 192 / 160 rows: 613 rows x 28672 186 / 172 /
+// 159 / 146, x 4096 of K 14336 in 4 slices 75.5 / 75 / 71 / 67; 1000 x 28672 203 / 245 / 222 / 254;
+// 5760 x 4096 of K 14336 527 / 510 / 482 / 615.
+static int pgemm_height(int M, int per_row) {
+  int best = 4;
+  long long least = 0;
+  for (int mi = 4; mi >= 1; --mi) {
+    const int h = 128 + 32 * mi;
+    const long long tiles = (long long)((M + h - 1) / h) * per_row;
+    const long long cost = ((tiles + 255) / 256 * (195 + h)) * 153 + tiles * h;
+    if (mi == 4 || cost < least) best = mi, least = cost;
+  }
+  return best;
 }
 
 // epi 0: C [M, N] bf16; epi 1: C [M, N / 2] = silu(gate) * up (8-interleaved gate|up W);
@@ -379,20 +416,24 @@ int docqa_pgemm(const void* A, const void* W, void* C, float* P, int M, int N, i
   if (epi == EPI_PARTIAL ? P == nullptr : (C == nullptr || S != 1)) return -1;
   if (epi != EPI_BF16 && epi != EPI_GLU && epi != EPI_PARTIAL && epi != EPI_RELU2 && epi != EPI_GELU) return -1;
   if (!docqa_aligned16(A) || !docqa_aligned16(W) || !docqa_aligned16(epi == EPI_PARTIAL ? (void*)P : C)) return -1;
-  const int ntm = (M + BM - 1) / BM, ntn = N / BN;
+  const int ntn = N / BN;
+  const int mi = pgemm_height(M, ntn * S), ntm = (M + 127 + 32 * mi) / (128 + 32 * mi);
   const uint16_t *a = (const uint16_t*)A, *w = (const uint16_t*)W;
   uint16_t* c = (uint16_t*)C;
   const int grid = ntm * ntn * S, Ks = K / S;
-  if (epi == EPI_BF16)
-    pgemm_kernel<EPI_BF16><<<grid, 512, 0, s>>>(a, w, c, P, M, N, K, ntm, ntn, S, Ks);
-  else if (epi == EPI_RELU2)
-    pgemm_kernel<EPI_RELU2><<<grid, 512, 0, s>>>(a, w, c, P, M, N, K, ntm, ntn, S, Ks);
-  else if (epi == EPI_GELU)
-    pgemm_kernel<EPI_GELU><<<grid, 512, 0, s>>>(a, w, c, P, M, N, K, ntm, ntn, S, Ks);
-  else if (epi == EPI_GLU)
-    pgemm_kernel<EPI_GLU><<<grid, 512, 0, s>>>(a, w, c, P, M, N, K, ntm, ntn, S, Ks);
-  else
-    pgemm_kernel<EPI_PARTIAL><<<grid, 512, 0, s>>>(a, w, c, P, M, N, K, ntm, ntn, S, Ks);
+#define DOCQA_PGEMM(E)                                                                                \
+  do {                                                                                                \
+    if (mi == 1) pgemm_kernel<E, 1><<<grid, 512, 0, s>>>(a, w, c, P, M, N, K, ntm, ntn, S, Ks);       \
+    else if (mi == 2) pgemm_kernel<E, 2><<<grid, 512, 0, s>>>(a, w, c, P, M, N, K, ntm, ntn, S, Ks);  \
+    else if (mi == 3) pgemm_kernel<E, 3><<<grid, 512, 0, s>>>(a, w, c, P, M, N, K, ntm, ntn, S, Ks);  \
+    else pgemm_kernel<E, 4><<<grid, 512, 0, s>>>(a, w, c, P, M, N, K, ntm, ntn, S, Ks);               \
+  } while (0)
+  if (epi == EPI_BF16) DOCQA_PGEMM(EPI_BF16);
+  else if (epi == EPI_RELU2) DOCQA_PGEMM(EPI_RELU2);
+  else if (epi == EPI_GELU) DOCQA_PGEMM(EPI_GELU);
+  else if (epi == EPI_GLU) DOCQA_PGEMM(EPI_GLU);
+  else DOCQA_PGEMM(EPI_PARTIAL);
+#undef DOCQA_PGEMM
   DOCQA_CHECK_LAUNCH();
   return 0;
 }
