@@ -17,9 +17,11 @@
 // x, dt and z are loaded 8 tokens ahead.  A long prompt
 // is cut into chunks that run side by side -- chunk states from zero, a carry pass over the
 // chunks, then the scan proper from each chunk's true entry state -- because one sequence's
-// channels alone (8192 = 128 waves) leave most of the 1024 SIMDs idle.
+// channels alone (8192 = 128 waves) leave most of the 1024 SIMDs idle.  Up to 16 states a channel is
+// spread over 4 or 8 lanes instead, which fills them without cutting (scan_lanes_kernel).
 #include "docqa_common.h"
 #include "docqa_elem.h"
+#include <type_traits>
 
 using namespace docqa;
 
@@ -203,11 +205,20 @@ struct ScanArgs {
   int C, N, Np, chunk, nchunk;
 };
 
+// CPL consecutive elements as they lie in memory
+template <typename T, int CPL>
+struct __attribute__((aligned(sizeof(T) * CPL))) Raw {
+  T e[CPL];
+};
+
 // LOCAL: the chunk's state from zero and its sum of dt (all chunks but a sequence's last).
 // Otherwise the scan proper, entering from the carried state (chunk 0) or the carry pass.
 // CPL: channels per lane -- two share a token's loads, address arithmetic and B / C reads.
+// Bound by its vector instructions (LOCAL: two products, an exp2 and an fma a state and token; the scan
+// proper one fma more).  Three workgroups a CU where the states' registers leave room: 816 of them, two
+// prompts of 1500 and 2500 tokens in chunks of 79, 377 -> 360 us.
 template <typename T, int NS, int LPC, int CPL, bool LOCAL>
-__global__ __launch_bounds__(256) void selective_scan_kernel(ScanArgs a) {
+__global__ __launch_bounds__(256, sizeof(T) * NS * CPL <= 64 ? 3 : 2) void selective_scan_kernel(ScanArgs a) {
   constexpr int NSP = NS * LPC, CB = 256 / LPC * CPL;
   __shared__ __attribute__((aligned(16))) float sbc[2][TB][2 * NSP];
   const int b = blockIdx.z, ck = blockIdx.y;
@@ -257,15 +268,17 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(ScanArgs a) {
     }
   };
   // x, dt, z of UB tokens from t (clamped: a token past the end is computed with dt = 0, which
-  // leaves the state alone, and stores nothing); row pointers are uniform, lanes add a column
-  float xn[UB][CPL], dn[UB][CPL], zn[UB][CPL];
+  // leaves the state alone, and stores nothing), as loaded: half the registers of their floats;
+  // row pointers are uniform, lanes add a column
+  using R = Raw<T, CPL>;
+  R xn[UB], dn[UB], zn[UB];
   auto fetch = [&](int t0) {
 #pragma unroll
     for (int i = 0; i < UB; ++i) {
       const size_t r = q0 + min(t0 + i, t_end - 1);
-      ldv<CPL>(X + r * a.C + (unsigned)cc, xn[i]);
-      ldv<CPL>(DT + r * a.C + (unsigned)cc, dn[i]);
-      if constexpr (!LOCAL) ldv<CPL>(Z + r * a.ld_z + (unsigned)cc, zn[i]);
+      xn[i] = *reinterpret_cast<const R*>(X + r * a.C + (unsigned)cc);
+      dn[i] = *reinterpret_cast<const R*>(DT + r * a.C + (unsigned)cc);
+      if constexpr (!LOCAL) zn[i] = *reinterpret_cast<const R*>(Z + r * a.ld_z + (unsigned)cc);
     }
   };
   stage(t_beg, 0);
@@ -275,25 +288,26 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(ScanArgs a) {
     __syncthreads();
     if (t0 + TB < t_end) stage(t0 + TB, buf ^ 1);
 #pragma unroll 1
-    for (int u = 0; u < TB; u += UB) {
-      float xv[UB][CPL], dv[UB][CPL], zv[UB][CPL];
+    for (int u = 0; u < TB && t0 + u < t_end; u += UB) {
+      R xr[UB], zr[UB];
+      float dv[UB][CPL];
 #pragma unroll
-      for (int i = 0; i < UB; ++i)
+      for (int i = 0; i < UB; ++i) {
+        xr[i] = xn[i];
+        if constexpr (!LOCAL) zr[i] = zn[i];
 #pragma unroll
-        for (int j = 0; j < CPL; ++j) {
-          xv[i][j] = xn[i][j];
-          dv[i][j] = t0 + u + i < t_end ? softplus_f(dn[i][j] + db[j]) : 0.f;
-          if constexpr (!LOCAL) zv[i][j] = silu_fast(zn[i][j]);
-        }
+        for (int j = 0; j < CPL; ++j) dv[i][j] = t0 + u + i < t_end ? softplus_f(ld1(&dn[i].e[j]) + db[j]) : 0.f;
+      }
       fetch(t0 + u + UB);
 #pragma unroll
       for (int i = 0; i < UB; ++i) {
         const float* Bt = &sbc[buf][u + i][l * NS];
         const float* Ct = &sbc[buf][u + i][NSP + l * NS];
-        float y[CPL];
+        float y[CPL], xv[CPL];
 #pragma unroll
         for (int j = 0; j < CPL; ++j) {
-          const float d = dv[i][j], dx = d * xv[i][j];
+          xv[j] = ld1(&xr[i].e[j]);
+          const float d = dv[i][j], dx = d * xv[j];
           y[j] = 0.f;
 #pragma unroll
           for (int n = 0; n < NS; ++n) {
@@ -307,7 +321,7 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(ScanArgs a) {
           for (int j = 0; j < CPL; ++j) {
 #pragma unroll
             for (int o = 1; o < LPC; o <<= 1) y[j] += __shfl_xor(y[j], o, 64);
-            y[j] = (y[j] + Dc[j] * xv[i][j]) * zv[i][j];
+            y[j] = (y[j] + Dc[j] * xv[j]) * silu_fast(ld1(&zr[i].e[j]));
           }
           if (l == 0 && ok && t0 + u + i < t_end)
             stv<CPL>((T*)a.y + (size_t)(q0 + t0 + u + i) * a.C + (unsigned)c, y);
@@ -329,7 +343,157 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(ScanArgs a) {
   }
 }
 
-// chunk k's entry state: decay over chunk k - 1 times its own entry state, plus the local one
+// The scan proper of whole sequences of at most 16 states with LPC lanes a channel: a sequence's channels are
+// then C LPC / 64 waves (8192 channels and 8 lanes: one a SIMD), every decay is computed once, and no chunk
+// states exist.  What a token and channel need only once (softplus, dt x, the gate) is done for TB tokens at
+// a time by all threads, through LDS; a channel's sums meet over its lanes by DPP, and lane i of LPC keeps
+// token i's, so the results leave through LDS as rows.  One barrier a TB tokens.  Bound by instruction
+// issue: 448 a 16 tokens, 36 of them exp2 at four times the cost.  8192 channels, us in chunks / so: 100
+// tokens 70 / 11, 1000 130 / 71, 4096 300 / 286, 1500 + 2500 377 / 228, 8 x 500 301 / 143.
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+// the sum of y[i] over a channel's LPC lanes, in lane i of them: each step halves the values and the lanes
+template <int LPC>
+__device__ __forceinline__ float lane_sums(const float (&y)[LPC], int l) {
+  static_assert(LPC == 4 || LPC == 8, "lanes a channel");
+  auto join = [&](float a, float b, bool hi, auto ctrl) { return (hi ? b : a) + dpp<decltype(ctrl)::value>(hi ? a : b); };
+  float q[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if constexpr (LPC == 8) q[i] = join(y[i], y[i + 4], l & 4, std::integral_constant<int, 0x141>{});   // lane 7 - l
+    else q[i] = y[i];
+  }
+  const float r0 = join(q[0], q[1], l & 1, std::integral_constant<int, 0xB1>{}),                      // lane l ^ 1
+              r1 = join(q[2], q[3], l & 1, std::integral_constant<int, 0xB1>{});
+  return join(r0, r1, l & 2, std::integral_constant<int, 0x4E>{});                                    // lane l ^ 2
+}
+template <typename T, int LPC>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void scan_lanes_kernel(ScanArgs a) {
+  constexpr int NS = 16 / LPC, CB = 256 / LPC, PAIRS = CB / 2, IT = TB * PAIRS / 256, PITCH = CB + 64 / LPC;
+  __shared__ __attribute__((aligned(16))) float2 sd[2][TB][CB];             // dt, dt x
+  __shared__ __attribute__((aligned(16))) float sbc[2][TB][LPC][2 * NS];    // a lane's B, then C
+  __shared__ __attribute__((aligned(16))) float sy[2][TB][PITCH];
+  const int b = blockIdx.y, q0 = a.cu[b], L = a.cu[b + 1] - q0;
+  if (L <= 0) return;
+  const int tid = threadIdx.x, cl = tid / LPC, l = tid % LPC, c0 = blockIdx.x * CB, c = c0 + cl;
+  const bool ok = c < a.C;
+  const int slot = a.slots[b];
+  const T *X = (const T*)a.x, *DT = (const T*)a.dt, *bc = (const T*)a.bc, *Z = (const T*)a.z;
+  using R = Raw<T, 2>;
+
+  float A[NS], S[NS];
+  {
+    const float* s0 = a.ctx[b] > 0 && slot >= 0 ? a.state + ((size_t)slot * a.C + min(c, a.C - 1)) * a.Np : nullptr;
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      const int n = l * NS + i;
+      A[i] = n < a.N ? a.A2[(size_t)min(c, a.C - 1) * a.Np + n] : 0.f;
+      S[i] = s0 && n < a.N ? s0[n] : 0.f;
+    }
+  }
+  // this thread's channel pair and tokens of a block, ahead of and behind the scan
+  const int p = tid % PAIRS, cp = min(c0 + 2 * p, a.C - 2);
+  const float D0 = a.D[cp], D1 = a.D[cp + 1], db0 = a.dt_b[cp], db1 = a.dt_b[cp + 1];
+  R xn[IT], dn[IT], zn[IT], xc[IT], zc[IT];
+  T bn[TB * 32 / 256];
+  // byte offsets of this thread's elements in a block's first TB rows; the rows' base is uniform
+  const uint32_t row = tid / PAIRS, rx = a.C * (uint32_t)sizeof(T), rz = a.ld_z * (uint32_t)sizeof(T),
+                 rb = a.ld_bc * (uint32_t)sizeof(T), ex = cp * (uint32_t)sizeof(T),
+                 eb = ((tid & 16 ? a.c_off : a.b_off) + min(tid & 15, a.N - 1)) * (uint32_t)sizeof(T);
+  const uint32_t ox = row * rx, oz = row * rz, ob = (tid >> 5) * rb;
+  auto fetch = [&](int t0) {               // past the end: the last token, used with dt = 0
+    const int tb = min(t0, L - 1);
+    const uint32_t last = min(L - 1 - tb, TB - 1);
+    const char *px = (const char*)X + (size_t)(q0 + tb) * rx, *pd = (const char*)DT + (size_t)(q0 + tb) * rx,
+               *pz = (const char*)Z + (size_t)(q0 + tb) * rz, *pb = (const char*)bc + (size_t)(q0 + tb) * rb;
+#pragma unroll
+    for (int k = 0; k < IT; ++k) {
+      const uint32_t o = min(ox + k * (256 / PAIRS) * rx, last * rx) + ex, oo = min(oz + k * (256 / PAIRS) * rz, last * rz) + ex;
+      xn[k] = *reinterpret_cast<const R*>(px + o);
+      dn[k] = *reinterpret_cast<const R*>(pd + o);
+      zn[k] = *reinterpret_cast<const R*>(pz + oo);
+    }
+#pragma unroll
+    for (int k = 0; k < TB * 32 / 256; ++k) bn[k] = *reinterpret_cast<const T*>(pb + (min(ob + k * 8 * rb, last * rb) + eb));
+  };
+  auto put = [&](int t0, int buf) {
+#pragma unroll
+    for (int k = 0; k < IT; ++k) {
+      const int tk = k * (256 / PAIRS) + tid / PAIRS;
+      const bool in = t0 + tk < L;
+      float d0 = softplus_f(ld1(&dn[k].e[0]) + db0), d1 = softplus_f(ld1(&dn[k].e[1]) + db1);
+      asm volatile("" : "+v"(d0), "+v"(d1));   // computed, then replaced: no branch around them
+      d0 = in ? d0 : 0.f;
+      d1 = in ? d1 : 0.f;
+      *reinterpret_cast<float4*>(&sd[buf][tk][2 * p]) = make_float4(d0, d0 * ld1(&xn[k].e[0]), d1, d1 * ld1(&xn[k].e[1]));
+    }
+#pragma unroll
+    for (int k = 0; k < TB * 32 / 256; ++k) {
+      const int n = tid & 15;
+      sbc[buf][k * 8 + (tid >> 5)][n / NS][(tid & 16 ? NS : 0) + n % NS] = n < a.N ? ld1(&bn[k]) : 0.f;
+    }
+  };
+  fetch(0);
+  put(0, 0);
+#pragma unroll
+  for (int k = 0; k < IT; ++k) xc[k] = xn[k], zc[k] = zn[k];
+  fetch(TB);
+  __syncthreads();
+  int buf = 0;
+  for (int t0 = 0; t0 < L; t0 += TB, buf ^= 1) {
+#pragma unroll
+    for (int h = 0; h < TB; h += LPC) {
+      float v[LPC][2 * NS], e[LPC][NS], y[LPC];
+      float2 d[LPC];
+#pragma unroll
+      for (int i = 0; i < LPC; ++i) {
+        d[i] = sd[buf][h + i][cl];
+        ldv<2 * NS>(sbc[buf][h + i][l], v[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < LPC; ++i)
+#pragma unroll
+        for (int n = 0; n < NS; ++n) e[i][n] = __builtin_amdgcn_exp2f(d[i].x * A[n]);
+#pragma unroll
+      for (int i = 0; i < LPC; ++i) {
+        y[i] = 0.f;
+#pragma unroll
+        for (int n = 0; n < NS; ++n) {
+          S[n] = e[i][n] * S[n] + d[i].y * v[i][n];
+          y[i] += S[n] * v[i][NS + n];
+        }
+      }
+      sy[buf][h + l][cl] = lane_sums<LPC>(y, l);
+    }
+    // the next block's part after this one's reads of LDS, so that its arithmetic mixes with the scan's
+    R xw[IT], zw[IT];
+#pragma unroll
+    for (int k = 0; k < IT; ++k) xw[k] = xn[k], zw[k] = zn[k];
+    if (t0 + TB < L) put(t0 + TB, buf ^ 1);
+    fetch(t0 + 2 * TB);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < IT; ++k) {
+      const int tk = k * (256 / PAIRS) + tid / PAIRS;
+      if (t0 + tk < L && c0 + 2 * p < a.C) {
+        const float2 y = *reinterpret_cast<const float2*>(&sy[buf][tk][2 * p]);
+        const float o[2] = {(y.x + D0 * ld1(&xc[k].e[0])) * silu_fast(ld1(&zc[k].e[0])),
+                            (y.y + D1 * ld1(&xc[k].e[1])) * silu_fast(ld1(&zc[k].e[1]))};
+        stv<2>((T*)((char*)a.y + (size_t)(q0 + t0) * rx + (ox + k * (256 / PAIRS) * rx + ex)), o);
+      }
+      xc[k] = xw[k], zc[k] = zw[k];
+    }
+  }
+  if (!ok || slot < 0) return;
+#pragma unroll
+  for (int i = 0; i < NS; ++i)
+    if (l * NS + i < a.N) a.state[((size_t)slot * a.C + c) * a.Np + l * NS + i] = S[i];
+}
+
+// chunk k's entry state: decay over chunk k - 1 times its own entry state, plus the local one; the
+// chunks' loads are in flight U at a time (one by one, 32 chunks took 15 us of latency)
 __global__ __launch_bounds__(256) void scan_carry_kernel(ScanArgs a) {
   const int b = blockIdx.y, L = a.cu[b + 1] - a.cu[b];
   const int e = blockIdx.x * 256 + threadIdx.x;
@@ -338,10 +502,23 @@ __global__ __launch_bounds__(256) void scan_carry_kernel(ScanArgs a) {
   const float A = a.A2[e];
   const int slot = a.slots[b];
   float s = (a.ctx[b] > 0 && slot >= 0) ? a.state[(size_t)slot * a.C * a.Np + e] : 0.f;
-  for (int k = 1; k * a.chunk < L; ++k) {
-    const size_t o = ((size_t)b * a.nchunk + k) * a.C;
-    s = __builtin_amdgcn_exp2f(A * a.csum[o + c]) * s + a.cstate[o * a.Np + e];
-    a.cstate[o * a.Np + e] = s;
+  constexpr int U = 8;
+  const int last = (L - 1) / a.chunk;
+  const size_t row = (size_t)b * a.nchunk * a.C;
+  for (int k0 = 1; k0 <= last; k0 += U) {
+    float d[U], l[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const size_t o = row + (size_t)min(k0 + u, last) * a.C;
+      d[u] = a.csum[o + c];
+      l[u] = a.cstate[o * a.Np + e];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (k0 + u <= last) {
+        s = __builtin_amdgcn_exp2f(A * d[u]) * s + l[u];
+        a.cstate[(row + (size_t)(k0 + u) * a.C) * a.Np + e] = s;
+      }
   }
 }
 
@@ -501,6 +678,14 @@ template <typename T>
 int dispatch_scan(const ScanArgs& a, int B, hipStream_t s) {
   const bool pair = a.C % 2 == 0 && a.ld_z % 2 == 0 && docqa_aligned16(a.x) && docqa_aligned16(a.dt) &&
                     (reinterpret_cast<uintptr_t>(a.z) & 7) == 0 && docqa_aligned16(a.y);
+  if (pair && a.N <= 16 && a.nchunk == 1) {
+    // 8 lanes a channel until they are 6 waves a SIMD (8192 channels, us of 8 / 4 lanes: 5 x 512 tokens
+    // 104 / 112, 6 x 512 122 / 114, 32 x 512 588 / 509, where a lane a channel takes 560)
+    if ((long long)B * a.C < 6 * 8192) scan_lanes_kernel<T, 8><<<dim3((a.C + 31) / 32, B), 256, 0, s>>>(a);
+    else scan_lanes_kernel<T, 4><<<dim3((a.C + 63) / 64, B), 256, 0, s>>>(a);
+    DOCQA_CHECK_LAUNCH();
+    return 0;
+  }
   if (a.N <= 8) return pair ? launch_scan<T, 8, 1, 2>(a, B, s) : launch_scan<T, 8, 1, 1>(a, B, s);
   if (a.N <= 16) return pair ? launch_scan<T, 16, 1, 2>(a, B, s) : launch_scan<T, 16, 1, 1>(a, B, s);
   if (a.N <= 24) return launch_scan<T, 24, 1, 1>(a, B, s);
