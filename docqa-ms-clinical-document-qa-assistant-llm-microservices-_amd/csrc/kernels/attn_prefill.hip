@@ -52,6 +52,13 @@ __device__ __forceinline__ int v_off(int row, int ch) {
   return row * D + ((ch ^ (((row & 3) << 2) & (D / 8 - 1))) << 3);
 }
 
+// the larger of a lane's value and that of the lane 32 on: v_permlane32_swap leaves the lower halves in one
+// register and the upper ones in the other
+__device__ __forceinline__ float half_max(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
 // Paged K/V source for prefix-cached prefill: keys [0, ctx_start[b]) were computed by an
 // earlier request (shared prompt prefix, prefix-cache hit) and keys
 // [ctx_start[b], ctx_start[b] + L) were just written by the fused RoPE/cache kernel, so
@@ -74,8 +81,13 @@ struct PagedKV {
 // G = 4, WPH = 1 (32-row tiles, 4 waves): at most 256 VGPRs so that two workgroups share a
 // CU and one's prologue (Q, block ids, first K/V tile: three dependent round trips) runs
 // under the other's main loop -- unbounded, hipcc spends ~300 and keeps one per CU
+// Heads up to 64: four workgroups a CU (128 VGPRs), for sequences of two or three tiles are mostly waits
+// for the next one.  With that, softmax in four instructions a score, uniform tile bases and 16-byte
+// stores, us: 256 sequences of 60..180 tokens, 12 heads of 64, 93 -> 47 (their bytes take 39), 64 of
+// 90..512 102 -> 53; causal, 32 heads of 128 over 8, 613 tokens 34.6 -> 21.6, 32 x 80..300 66 -> 46,
+// 2048 106 -> 68
 template <int D, bool CAUSAL, bool PAGED, int G, int WPH, bool PFX = false>
-__global__ __launch_bounds__(64 * G * WPH, (G == 4 && WPH == 1) ? 2 : 1) void flash_prefill_kernel(
+__global__ __launch_bounds__(64 * G * WPH, D <= 64 ? 4 : G == 4 && WPH == 1 ? 2 : 1) void flash_prefill_kernel(
     const uint16_t* __restrict__ qkv, int row_stride, const int* __restrict__ cu_seqlens,
     uint16_t* __restrict__ out, int o_stride, int Hq, int Hkv, float scale, PagedKV pk,
     CascadeOut co) {
@@ -163,8 +175,15 @@ __global__ __launch_bounds__(64 * G * WPH, (G == 4 && WPH == 1) ? 2 : 1) void fl
   for (int i = 0; i < NDT; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
-  float m_run = -FLT_MAX, l_run = 0.f;
-  const float sl2 = scale * kLog2e;
+  float m_run = -FLT_MAX, l_run = 0.f;          // l_run: this half-wave's keys, joined at the end
+  // a negative scale turns Q's sign instead, a zero one is as good as this (and keeps -inf masks out of 0 x inf)
+  const float sl2 = fmaxf(fabsf(scale) * kLog2e, FLT_MIN);
+  if (scale < 0.f) {
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) qf[ks][j] = -qf[ks][j];
+  }
 
   const int kv_end = CAUSAL ? min(Lk, P0 + q_start + QBW) : Lk;
   const int ntiles = (kv_end + KB - 1) / KB;
@@ -185,22 +204,25 @@ __global__ __launch_bounds__(64 * G * WPH, (G == 4 && WPH == 1) ? 2 : 1) void fl
       __syncthreads();
     }
   }
+  static_assert(KB * NCH % NT == 0, "whole chunks a thread");
+  // this thread's first chunk of a tile; the others lie whole rows on, so their bases are uniform
+  const int row0 = tid / NCH, ch0 = tid % NCH;
+  const uint32_t voff = (uint32_t)row0 * (uint32_t)(row_stride * 2) + ch0 * 16;
   auto load_tile = [&](int t) {
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
-      const int idx = tid + NT * i;
-      const int row = idx / NCH, ch = idx % NCH;
-      const int key = t * KB + row;
-      if (idx < KB * NCH && key < Lk) {
+      const int first = t * KB + i * (NT / NCH);
+      if (row0 < Lk - first) {
         if constexpr (PAGED) {
+          const int key = first + row0;
           const int blk = bt_lds ? s_bt[key >> pk.log2BS]
                                  : pk.block_tables[(size_t)(PFX ? 0 : b) * pk.maxb + (key >> pk.log2BS)];
-          const size_t off = (((size_t)blk * Hkv + kvh) * pk.BS + (key & (pk.BS - 1))) * D + ch * 8;
+          const size_t off = (((size_t)blk * Hkv + kvh) * pk.BS + (key & (pk.BS - 1))) * D + ch0 * 8;
           rk[i] = *reinterpret_cast<const uint4*>(pk.k + off);
           rv[i] = *reinterpret_cast<const uint4*>(pk.v + off);
         } else {
-          rk[i] = *reinterpret_cast<const uint4*>(kbase + (size_t)key * row_stride + ch * 8);
-          rv[i] = *reinterpret_cast<const uint4*>(vbase + (size_t)key * row_stride + ch * 8);
+          rk[i] = *reinterpret_cast<const uint4*>((const char*)(kbase + (size_t)first * row_stride) + voff);
+          rv[i] = *reinterpret_cast<const uint4*>((const char*)(vbase + (size_t)first * row_stride) + voff);
         }
       } else {
         rk[i] = make_uint4(0, 0, 0, 0);
@@ -211,11 +233,9 @@ __global__ __launch_bounds__(64 * G * WPH, (G == 4 && WPH == 1) ? 2 : 1) void fl
   auto store_tile = [&]() {
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
-      const int idx = tid + NT * i;
-      if (idx >= KB * NCH) break;
-      const int row = idx / NCH, ch = idx % NCH;
-      *reinterpret_cast<uint4*>(sK + k_off<D>(row, ch)) = rk[i];
-      *reinterpret_cast<uint4*>(sV + v_off<D>(row, ch)) = rv[i];
+      const int row = row0 + i * (NT / NCH);
+      *reinterpret_cast<uint4*>(sK + k_off<D>(row, ch0)) = rk[i];
+      *reinterpret_cast<uint4*>(sV + v_off<D>(row, ch0)) = rv[i];
     }
   };
 
@@ -246,39 +266,42 @@ __global__ __launch_bounds__(64 * G * WPH, (G == 4 && WPH == 1) ? 2 : 1) void fl
           x[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[ks], x[kt], 0, 0, 0);
         }
       }
-      // ---- online softmax (log2 domain); keys on registers, query on lane
-      float mx = -FLT_MAX;
+      // ---- online softmax (log2 domain); keys on registers, query on lane.  The product of 32 x 32 x 16 is
+      // worth 32 clocks a KB of operands, so at D 64 these instructions are the longer part: only a tile that
+      // holds a masked key compares, and a score costs half a max, one fma, one exp2, one add.
+      if (kb + KB > Lk || (CAUSAL && kb + KB - 1 > P0 + q_wave)) {
+        const int lim = (CAUSAL ? min(Lk, P0 + my_q + 1) : Lk) - kb - 4 * hh;
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            x[kt][r] = kt * 32 + (r & 3) + 8 * (r >> 2) < lim ? x[kt][r] : -INFINITY;
+      }
+      float mx = -INFINITY;
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, x[kt][r]);
+      mx = half_max(mx);
+      const float m_new = fmaxf(m_run, mx * sl2);   // every key so far masked: stays -FLT_MAX, and p is 0
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      float rs[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const int key = kb + kt * 32 + (r & 3) + 8 * (r >> 2) + 4 * hh;
-          float s = x[kt][r] * sl2;
-          const bool masked = (key >= Lk) || (CAUSAL && key > P0 + my_q);
-          s = masked ? -FLT_MAX : s;
-          x[kt][r] = s;
-          mx = fmaxf(mx, s);
-        }
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      const float m_new = fmaxf(m_run, mx);
-      const bool dead = (m_new == -FLT_MAX);       // every key so far masked
-      const float alpha = dead ? 1.f : exp2f(m_run - m_new);
-      float rs = 0.f;
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float p = (dead || x[kt][r] == -FLT_MAX) ? 0.f : exp2f(x[kt][r] - m_new);
+          const float p = __builtin_amdgcn_exp2f(fmaf(x[kt][r], sl2, -m_new));
           x[kt][r] = p;
-          rs += p;
+          rs[r & 3] += p;
         }
-      rs += __shfl_xor(rs, 32, 64);
-      l_run = l_run * alpha + rs;
+      l_run = l_run * alpha + ((rs[0] + rs[1]) + (rs[2] + rs[3]));
+      if (__ballot(m_new != m_run)) {
+#pragma unroll
+        for (int i = 0; i < NDT; ++i)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[i][r] *= alpha;
+      }
       m_run = m_new;
-#pragma unroll
-      for (int i = 0; i < NDT; ++i)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[i][r] *= alpha;
 
       // ---- O^T += V^T P^T
 #pragma unroll
@@ -314,6 +337,7 @@ __global__ __launch_bounds__(64 * G * WPH, (G == 4 && WPH == 1) ? 2 : 1) void fl
     }
   }
 
+  l_run += __shfl_xor(l_run, 32, 64);
   if constexpr (PFX) {   // chunk partial: un-normalised O and (max, sum) per (row, head)
     // O^T is lane = query row, registers = dims: stored straight, every 16-B store lands in
     // a different row (32 partial 128-B lines per instruction).  Transpose each 32-dim
@@ -342,21 +366,22 @@ __global__ __launch_bounds__(64 * G * WPH, (G == 4 && WPH == 1) ? 2 : 1) void fl
       *reinterpret_cast<float2*>(co.ml + (((size_t)b * L + my_q) * Hq + h) * 2) = make_float2(m_run, l_run);
     return;
   }
-  // ---- epilogue: O[q][dim] = O^T[dim][q] / l
-  if (my_q < L) {
-    const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
-    uint16_t* op = out + (size_t)(seq0 + my_q) * o_stride + (size_t)h * D;
+  // ---- epilogue: O[q][dim] = O^T[dim][q] / l.  A lane holds 4 dims of every 8; two of its groups against
+  // the other half-wave's make 16-byte stores
+  const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
+  uint16_t* op = out + (size_t)(seq0 + my_q) * o_stride + (size_t)h * D;
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
+  for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        const int d0 = dt * 32 + 8 * g4 + 4 * hh;
-        uint2 v;
-        v.x = pack2(o[dt][4 * g4 + 0] * inv, o[dt][4 * g4 + 1] * inv);
-        v.y = pack2(o[dt][4 * g4 + 2] * inv, o[dt][4 * g4 + 3] * inv);
-        *reinterpret_cast<uint2*>(op + d0) = v;
-      }
-  }
+    for (int g4 = 0; g4 < 4; g4 += 2) {
+      const float* a = reinterpret_cast<const float*>(&o[dt]) + 4 * g4;
+      const auto lo = __builtin_amdgcn_permlane32_swap(pack2(a[0] * inv, a[1] * inv), pack2(a[4] * inv, a[5] * inv),
+                                                       false, false);
+      const auto hi = __builtin_amdgcn_permlane32_swap(pack2(a[2] * inv, a[3] * inv), pack2(a[6] * inv, a[7] * inv),
+                                                       false, false);
+      if (my_q < L)
+        *reinterpret_cast<uint4*>(op + dt * 32 + 8 * (g4 + hh)) = make_uint4(lo[0], hi[0], lo[1], hi[1]);
+    }
 }
 }  // namespace
 
