@@ -22,6 +22,7 @@
 // Shapes: N % 128 == 0, K % 64 == 0, any M.
 #include "docqa_asm.h"
 #include "docqa_common.h"
+#include <type_traits>
 
 using namespace docqa;
 
@@ -176,7 +177,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(const uint16_t* __restrict__ 
 // (bge-base, 30720 rows, us of QKV / O / FFN up / down: 146 / 54 / 226 / 173; here 119 / 49 / 175 /
 // 140, 0.9 to 1.05 PFLOP/s, the matrix cores busy 45 % of the time at the 1.9 GHz this load runs at,
 // the rest in the latency of units and epilogues).
-// Here a wave owns 128 rows x 64 columns (v_mfma_f32_32x32x16_bf16: 48 KB for 1024 clocks), and a
+// Here a wave owns 128 rows x 64 columns (96, with half an HA1, on 192-row tiles) (v_mfma_f32_32x32x16_bf16: 48 KB for 1024 clocks), and a
 // workgroup's epilogue runs under the other one's products.
 //   * K-tiles of 64 come as three units of 128 rows x 64 (whole 128-byte lines: with 64-byte rows
 //     LDS-DMA moves 15 TB/s over the chip, with 128-byte ones 20 to 29) through a ring of five:
@@ -190,16 +191,18 @@ __global__ __launch_bounds__(256) void gemm_kernel(const uint16_t* __restrict__ 
 //   * the tile is put together in LDS (16-B chunk ^ (row & 15): 32 rows' pieces hit distinct
 //     banks) and stored in whole rows; the residual comes into the same places by LDS-DMA first
 //     and is added in fp32 before the one rounding.
-constexpr int WM = 256, WN = 128;
+constexpr int WN = 128;
 constexpr int UNIT = 128 * BK * 2, NUNIT = 5;         // 16 KB units of the ring, 80 KB
 
-template <int EPI>
+template <int EPI, int WM>
 __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ W,
                                                            const uint16_t* __restrict__ bias,
                                                            const uint16_t* __restrict__ res, uint16_t* __restrict__ C,
                                                            int M, int N, int K) {
   __shared__ __attribute__((aligned(16))) char smem[NUNIT * UNIT];
   static_assert(NUNIT * UNIT >= WM * WN * 2, "epilogue tile");
+  constexpr int WR = WM / 2, M1 = WR / 32 - 2, L1 = 2 * M1;   // a wave row; 32-row tiles and loads a thread of its HA1
+  static_assert(M1 == 1 || M1 == 2, "192 or 256 rows");
   const int nbn = N / WN;
   const int wg = xcd_remap(blockIdx.x, gridDim.x);
   const int row0 = (wg / nbn) * WM, col0 = (wg % nbn) * WN;
@@ -218,15 +221,17 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(const uint16_t* __res
     const int r = i * 32 + (tid >> 3);
     boff[i] = (uint32_t)r * (uint32_t)(K * 2) + lch;
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-      aoff[h][i] = (uint32_t)min((r >> 6) * 128 + h * 64 + (r & 63), M - 1 - row0) * (uint32_t)(K * 2) + lch;
+    for (int h = 0; h < 2; ++h) {
+      const int hr = h ? 32 * M1 : 64;               // rows of this half of a wave row
+      aoff[h][i] = (uint32_t)min(r / hr * WR + h * 64 + r % hr, M - 1 - row0) * (uint32_t)(K * 2) + lch;
+    }
   }
   // unit `part` (0 HA0, 1 HB, 2 HA1) of K-tile kt into ring slot `slot`
   auto issue = [&](int part, int kt, int slot) {
     const uint32_t d = lds + (uint32_t)(slot * UNIT + wave * 1024);
     const uint32_t k = (uint32_t)kt * (BK * 2);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < (part == 2 ? L1 : 4); ++i)
       glds16_off(part == 1 ? wb : ab, (part == 1 ? boff[i] : aoff[part >> 1][i]) + k,
                  __builtin_amdgcn_readfirstlane(d + i * 4096));
   };
@@ -239,15 +244,16 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(const uint16_t* __res
     return *reinterpret_cast<const bf16x8*>(smem + slot * UNIT + row * 128 + ((ch ^ ((row >> 1) & 7)) << 4));
   };
 
-  f32x16 acc[2][4];
+  f32x16 acc[2][2 + M1];
 #pragma unroll
   for (int n = 0; n < 2; ++n)
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
+    for (int m = 0; m < 2 + M1; ++m)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[n][m][r] = 0.f;
   bf16x8 w[4][2];                                    // [16-deep k-step][n-tile] of the current K-tile
-  auto phase = [&](int slot_a, int slot_b, bool first) {
+  auto phase = [&](int slot_a, int slot_b, auto part) {
+    constexpr bool first = decltype(part)::value;
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       if (first) {
@@ -256,9 +262,9 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(const uint16_t* __res
       }
       bf16x8 a[2];
 #pragma unroll
-      for (int m = 0; m < 2; ++m) a[m] = frag(slot_a, wr * 64 + m * 32 + l32, ks * 2 + hh);
+      for (int m = 0; m < (first ? 2 : M1); ++m) a[m] = frag(slot_a, wr * (first ? 64 : 32 * M1) + m * 32 + l32, ks * 2 + hh);
 #pragma unroll
-      for (int m = 0; m < 2; ++m)
+      for (int m = 0; m < (first ? 2 : M1); ++m)
 #pragma unroll
         for (int n = 0; n < 2; ++n) {
           f32x16& c = acc[n][first ? m : 2 + m];
@@ -275,23 +281,23 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(const uint16_t* __res
   int s0 = 0;                                        // slot of unit 3t
   auto slot = [&](int k) { return s0 + k < NUNIT ? s0 + k : s0 + k - NUNIT; };   // of unit 3t + k, k <= 4
   for (int t = 0; t < nk - 1; ++t) {
-    wait_vmcnt<8>();
+    wait_vmcnt<4 + L1>();
     open();
     issue(1, t + 1, slot(4));
-    phase(slot(0), slot(1), true);
+    phase(slot(0), slot(1), std::true_type{});
     wait_vmcnt<8>();
     open();
     issue(2, t + 1, slot(0));
     if (t + 2 < nk) issue(0, t + 2, slot(1));
-    phase(slot(2), 0, false);
+    phase(slot(2), 0, std::false_type{});
     s0 = slot(3);
   }
-  wait_vmcnt<4>();
+  wait_vmcnt<L1>();
   open();
-  phase(slot(0), slot(1), true);
+  phase(slot(0), slot(1), std::true_type{});
   wait_vmcnt<0>();
   open();
-  phase(slot(2), 0, false);
+  phase(slot(2), 0, std::false_type{});
   open();                                            // the ring is the epilogue's tile now
 
   // 16-B chunk of the tile that piece `it` of this thread is: row 16 it + tid / 16
@@ -299,7 +305,7 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(const uint16_t* __res
   if constexpr (EPI == EPI_BIAS_RES) {
     const char* rb = (const char*)(res + (size_t)row0 * N + col0);
 #pragma unroll
-    for (int it = 0; it < 16; ++it)
+    for (int it = 0; it < WM / 16; ++it)
       glds16_off(rb, (uint32_t)min(16 * it + prow, M - 1 - row0) * (uint32_t)(N * 2) + pcol * 2,
                  __builtin_amdgcn_readfirstlane(lds + it * 4096 + wave * 1024));
     wait_vmcnt<0>();
@@ -313,8 +319,8 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(const uint16_t* __res
       float b[4] = {0.f, 0.f, 0.f, 0.f};
       if constexpr (EPI != EPI_NONE) add4(b, *reinterpret_cast<const uint2*>(bias + col0 + col));
 #pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        const int row = wr * 128 + m * 32 + l32;
+      for (int m = 0; m < 2 + M1; ++m) {
+        const int row = wr * WR + m * 32 + l32;
         uint2* at = reinterpret_cast<uint2*>(smem + row * 256 + (((col >> 3) ^ (row & 15)) << 4) + (hh << 3));
         float v[4];
 #pragma unroll
@@ -330,7 +336,7 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(const uint16_t* __res
   __syncthreads();
   uint16_t* out = C + (size_t)row0 * N + col0 + pcol;
 #pragma unroll
-  for (int it = 0; it < 16; ++it) {
+  for (int it = 0; it < WM / 16; ++it) {
     const int r = 16 * it + prow;
     const uint4 v = *reinterpret_cast<const uint4*>(smem + it * 4096 + tid * 16);
     if (row0 + r < M) *reinterpret_cast<uint4*>(out + (size_t)r * N) = v;
@@ -466,6 +472,15 @@ __global__ __launch_bounds__(256, 2) void gemm_few_kernel(const uint16_t* __rest
 }
 }  // namespace
 
+// What `tiles` ring tiles take, in eighths of a round of 512 (two workgroups a CU): alone on its CU a workgroup
+// takes five of them.  A round of 192-row tiles is worth 0.8 of one of 256 (fitted to 95 launches, bge-base and
+// MiniLM at 3600..34000 rows: 0.3 % off the better one on average, 256 rows alone 7 %; us of 256 / 192: QKV
+// 4500 rows 25.6 / 21.4, down 22000 rows 129 / 107, up 13000 rows 79 / 85)
+static long long ring_cost(long long tiles) {
+  const long long rest = tiles % 512;
+  return tiles / 512 * 8 + (rest == 0 ? 0 : rest <= 256 ? 5 : 8);
+}
+
 int docqa_gemm(const void* A, const void* W, const void* bias, const void* res, void* C, int M,
                int N, int K, int epi, hipStream_t s) {
   if (M == 0) return 0;
@@ -480,7 +495,10 @@ int docqa_gemm(const void* A, const void* W, const void* bias, const void* res, 
   // rows, 288 workgroups, 5.7 / 6.3, 256 rows, 576 of them, 8.0 / 6.5), 64 x 64 up to three (64 / 128
   // wide: QKV 1024 rows, 576, 13.6 / 14.4, 1500 rows, 864, 16.6 / 14.7; O 4096 rows, 768, 13.2 / 13.5),
   // 256 x 128 from one on (128 wide / ring: QKV 4096 rows, 288, 28.1 / 25.0, 30720 rows 146 / 119;
-  // FFN down, K 3072, 8192 rows, 192, 48.6 / 54.2, 19000 rows, 450, 103 / 91).  Row offsets inside
+  // FFN down, K 3072, 8192 rows, 192, 48.6 / 54.2, 19000 rows, 450, 103 / 91), of them 192 rows where
+  // those end in less (see ring_cost), and where a workgroup a CU holds them but not the 128 x 128 tiles
+  // (QKV 2600 rows 17.6 / 14.6, O 7000 rows 17.5 / 15.1; with 128-wide tiles below that too, or 192-row
+  // tiles above it, 128 x 128 wins: O 5200 rows 13.4 / 14.1, 10500 rows 19.1 / 21.5).  Row offsets inside
   // those tiles are 32-bit
   auto tiles = [&](int tm, int tn) { return (long long)((M + tm - 1) / tm) * (N / tn); };
 #define DOCQA_GEMM_EPI(KERNEL, GRID)                                                             \
@@ -493,16 +511,19 @@ int docqa_gemm(const void* A, const void* W, const void* bias, const void* res, 
   } while (0)
 #define DOCQA_FEW32(E) gemm_few_kernel<32, E>
 #define DOCQA_FEW64(E) gemm_few_kernel<64, E>
-#define DOCQA_RING(E) gemm_ring_kernel<E>
+#define DOCQA_RING(E) gemm_ring_kernel<E, 256>
+#define DOCQA_RING192(E) gemm_ring_kernel<E, 192>
   if (epi < EPI_NONE || epi > EPI_GLU) return -1;
-  if (epi != EPI_GLU && (long long)WM * (K > N ? K : N) * 2 < (1ll << 32)) {
+  if (epi != EPI_GLU && 256ll * (K > N ? K : N) * 2 < (1ll << 32)) {
     int kind = 0;
     if (K % 128 == 0 && tiles(32, 32) <= 512) kind = 32;
     else if (tiles(64, 64) <= 768) kind = 64;
-    else if (tiles(WM, WN) >= 256) kind = WM;
+    else if (tiles(256, WN) >= 256) kind = ring_cost(tiles(192, WN)) * 4 < ring_cost(tiles(256, WN)) * 5 ? 192 : 256;
+    else if (nwg > 256 && tiles(192, WN) <= 256) kind = 192;
     if (kind == 32) DOCQA_GEMM_EPI(DOCQA_FEW32, tiles(32, 32));
     else if (kind == 64) DOCQA_GEMM_EPI(DOCQA_FEW64, tiles(64, 64));
-    else if (kind) DOCQA_GEMM_EPI(DOCQA_RING, tiles(WM, WN));
+    else if (kind == 192) DOCQA_GEMM_EPI(DOCQA_RING192, tiles(192, WN));
+    else if (kind) DOCQA_GEMM_EPI(DOCQA_RING, tiles(256, WN));
     if (kind) {
       DOCQA_CHECK_LAUNCH();
       return 0;

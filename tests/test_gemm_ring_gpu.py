@@ -11,6 +11,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [
     (256 * 128, 256, 64), (256 * 127 + 1, 256, 128), (256 * 85 + 255, 384, 192), (256 * 86 - 31, 384, 320),
     (256 * 28 + 129, 1152, 384), (256 * 14 + 37, 2304, 768), (256 * 43 + 5, 768, 3072),
+    # 192-row tiles of the ring, in one round and in more
+    (4500, 2304, 64), (192 * 23 - 1, 2304, 192), (192 * 114 + 5, 768, 128), (192 * 14 - 60, 2304, 320), (2689, 2304, 768),
     # 32 x 32 and 64 x 64 tiles (K not a multiple of 128: the latter), 1 .. 6 stages, one row
     (1, 128, 128), (24, 384, 256), (33, 1152, 384), (128, 768, 512), (31, 128, 640), (1, 128, 64), (65, 256, 192),
     (300, 2304, 768), (1000, 768, 3072), (700, 3072, 320), (129, 128, 448),
