@@ -23,8 +23,8 @@
 //     and no separate silu_mul launch.  7 n-tiles per workgroup (112 rows) make the Llama-3-8B
 //     shape exactly 256 workgroups = one per CU, and halve the L2 traffic of re-reading X
 //     per workgroup (at M = 64 that X traffic, not HBM, was the limiter).
-// That kernel (dgemm_kernel) serves up to 16 rows, where its sums are also the fused-norm forms' bit for
-// bit, and 129..192 rows (64-row weight tiles, three m-tiles per wave, no fused SwiGLU); 17..128 rows take
+// That kernel (dgemm_kernel) serves up to 4 rows, where its sums are also the fused-norm forms' bit for
+// bit, and 129..192 rows (64-row weight tiles, three m-tiles per wave, no fused SwiGLU); 5..128 rows take
 // dstream_kernel below, whose X rows come through the LDS ring as well.
 // Shapes: N % (16 NT) == 0, (K / S) % 512 == 0 (whole 4-stage ring turns).
 #include "docqa_common.h"
@@ -37,6 +37,7 @@
 using namespace docqa;
 
 namespace {
+constexpr int kNormRows = 4;   // rows of the fused residual + RMSNorm forms
 constexpr int BN = 64, BKD = 128, NS = 4, MR = 192;   // NS: default ring slots, K granule 4 stages
 constexpr int KSTEPS = BKD / 32;               // 16x16x32 k-steps per stage
 enum { EPI_BF16 = 0, EPI_PARTIAL = 1, EPI_GLU = 2, EPI_ARGMAX = 3, EPI_RELU2 = 4, EPI_GELU = 5 };
@@ -481,7 +482,7 @@ __global__ __launch_bounds__(256) void dgemm_kernel(const uint16_t* __restrict__
 }
 
 // ---------------------------------------------------------------------------------------
-// 17..128 rows: X and W tiles through one LDS ring, TM X rows x TN weight rows x one K slice a workgroup.
+// 5..128 rows: X and W tiles through one LDS ring, TM X rows x TN weight rows x one K slice a workgroup.
 // Such a product is bound by what a CU can fetch: its weights once from HBM and X again for every TN
 // weight rows from L2, so both arrive as whole 128-byte lines straight into LDS (as MFMA fragments read
 // into registers, 64 bytes a row, X cost as much as W: 128 rows of 28672 x 4096 59 us, so 52; of
@@ -737,21 +738,23 @@ static void launch_glu7(int mt, dim3 grid, hipStream_t s, const uint16_t* x, con
   else dgemm_kernel<EPI_GLU, 8, 7, NS><<<grid, 256, 0, s>>>(x, w, y, nullptr, M, N, K, K, 0);
 }
 
-// N % 64 == 0.  Up to 16 rows and 129..192: the ring of weights alone.  Between them X goes through the
+// N % 64 == 0.  Up to 4 rows and 129..192: the ring of weights alone.  Between them X goes through the
 // ring too, on the X rows' next power of two x 64 weight rows; us of 64 / 128 weight rows for 128 rows, and
 // of two / three workgroups a CU for 32 rows, by what fills the chip:
 //   128 rows: 500 and 448 workgroups of 64 (N 32000 and 28672 x K 4096) 67.8 / 61.3 and 63.2 / 52.9, 384
 //     (6144 x 4096 S 4) 20.1 / 17.9; 256 of 64 (16384 x 4096) 36.4 / 39.1, (4096 x 4096 S 4) 12.2 / 15;
 //   32 rows: 500 and 448 of them 51.5 / 48.1 and 45.6 / 44.2, 192 (6144 x 4096 S 2) 12.7 / 13.2.
+// At 16 rows those 32-row tiles still gain over the weights' ring: 32000 x 4096 52 / 49.7, gate|up 44.1 / 41.7,
+// O 8.5 / 8.0, down 20.2 / 19.8, QKV 11.9 / 12.1.
 // (With 8 waves on 128 x 128 tiles, 2 x 4 or two groups along k: 52.7 - 53.8 for 52.9.)
 template <int EPI>
 static void launch_rows(dim3 grid, hipStream_t s, const uint16_t* x, const uint16_t* w, uint16_t* y, float* p, int M,
                         int N, int K, int Ks, float* pv = nullptr, int* pi = nullptr, int nv = 0) {
   const int mt = (M + 15) / 16;
   int xr = remap_slices(grid);
-  if (mt == 1) {
+  if (M <= kNormRows) {
     dgemm_kernel<EPI, 1, 4, NS><<<grid, 256, 0, s>>>(x, w, y, p, M, N, K, Ks, xr, pv, pi, nv);
-  } else if (mt == 2) {
+  } else if (mt <= 2) {
     if (grid.x * grid.y > 256)
       dstream_kernel<EPI, 32, 64, 1, 1, 4, 3><<<grid, 256, 0, s>>>(x, w, y, p, M, N, K, Ks, xr, pv, pi, nv);
     else
@@ -821,7 +824,6 @@ int docqa_dgemm_partial(const void* X, const void* W, float* P, int M, int N, in
 // Few-row split-K projection with the residual add + RMSNorm fused in (NormArgs): P [S, M, N]
 // fp32 slabs (scratch), residual [M, N] updated, out [M, N] = rmsnorm(residual) * gamma.
 // M <= kNormRows, N <= 8192 (4 chunks of 8 per lane), 64-row weight tiles.
-constexpr int kNormRows = 4;
 int docqa_dgemm_add_rmsnorm(const void* X, const void* W, float* P, int M, int N, int K, int S, void* residual,
                             const void* gamma, void* out, float eps, int* tick, hipStream_t s) {
   if (M == 0) return 0;
@@ -878,11 +880,11 @@ int docqa_dgemm_glu(const void* X, const void* W, void* Y, int M, int N, int K, 
   if (M > 128) return -1;
   const uint16_t* x = (const uint16_t*)X;
   const uint16_t* w = (const uint16_t*)W;
-  // 112-row tiles of the weight ring up to 16 rows and at 33..64 (28672 x 4096, 64 rows: 47.4 us, 64 x 64
+  // 112-row tiles of the weight ring up to 4 rows and at 33..64 (28672 x 4096, 64 rows: 47.4 us, 64 x 64
   // tiles 52.2, 64 x 128 of two k-groups 47.3; 32 rows 45.6 - 47.2 against 44.2) and where N has no 64-row tiles
   const bool wide = shape_ok(M, N, K, 1, 112) && N / 112 >= 192, even = shape_ok(M, N, K, 1, BN);
   const int mt = (M + 15) / 16;
-  if (wide && (!even || mt == 1 || mt == 3 || mt == 4))
+  if (wide && (!even || M <= kNormRows || mt == 3 || mt == 4))
     launch_glu7(mt, dim3(N / 112), s, x, w, (uint16_t*)Y, M, N, K);
   else if (even)
     launch_rows<EPI_GLU>(dim3(N / BN), s, x, w, (uint16_t*)Y, nullptr, M, N, K, K);

@@ -188,7 +188,7 @@ def decode_plan(M: int, N: int, K: int) -> tuple[int, int]:
     64-row tiles with the smallest split giving >= 192 workgroups; at 65-128 rows 128-row
     tiles (X re-read from L2 half as often) where such a split exists (QKV S=4: 21.9 us vs
     hipBLASLt 25.2 at M=128; O S=8: 17.2 vs 24.4), else 64-row tiles (down S=4: 40.7 vs 75.1).
-    With X through the LDS ring (17..128 rows, the width then chosen at the launch) the same plans
+    With X through the LDS ring (5..128 rows, the width then chosen at the launch) the same plans
     take QKV 17.9, O at S=4 12.2 and down 31.8 us at M=128; QKV 14.9, O 9.5 and down 23.9 at M=64."""
     if M > 192 or N % 64 or N >= 65536 or (N >= 16384 and M > 32):
         return 0, 64

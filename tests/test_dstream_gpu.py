@@ -1,4 +1,4 @@
-"""The 17..128-row decode products: every tile and epilogue at the edges of its rows, against 64-bit products.
+"""The 5..128-row decode products: every tile and epilogue at the edges of its rows, against 64-bit products.
 
 A fp32 sum of K terms of bf16 x bf16 (exact in fp32) differs from the true one by at most K 2^-24 sum |x w|,
 whatever its order; a bf16 result by half an ulp (2^-9 of the value, 2^-8 where it rounds up a binade) more."""
@@ -7,7 +7,7 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-ROWS = [16, 17, 31, 32, 33, 64, 65, 97, 128]
+ROWS = [4, 5, 16, 17, 31, 32, 33, 64, 65, 97, 128]
 # N, K, S: one tile of either width; an odd count; more than two workgroups a CU; 128-wide tiles; slices
 SHAPES = [(64, 512, 1), (128, 1024, 2), (192, 512, 1), (16640, 512, 1), (24576, 512, 1), (6144, 2048, 4), (320, 4096, 8)]
 
