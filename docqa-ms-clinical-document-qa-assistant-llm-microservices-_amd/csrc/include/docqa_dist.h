@@ -9,11 +9,14 @@
 //              rows past n, NaN and +inf are FLT_MAX, "missing" to the selection
 //   row-major  D[q][row], no minima
 //
-// Two kernels.  knn_dist_kernel: 128 rows x QT queries a workgroup through an LDS-DMA ring.
+// Three kernels.  knn_dist_kernel: 128 rows x QT queries a workgroup through an LDS-DMA ring.
 // fp32 runs on v_mfma_f32_32x32x2_f32 (256 flops a clock and CU: 154 TFLOP/s measured), so a
 // 64 x 64 wave tile needs 4 ds_read_b128 per 16 MFMAs of 64 clocks and is bound by the matrix
-// cores from 64 queries on (250000 x 768 by 256 queries: 778 us, 126 TFLOP/s); QT = 32 keeps one
-// query tile a wave and is bound by the database's bytes (the same by 1 query: 134 us, 5.7 TB/s).  knn_dist_small_kernel: 32 rows x 32 queries a workgroup with K split over
+// cores from 64 queries on; QT = 32 keeps one query tile a wave and is bound by the database's bytes
+// (250000 x 768 by 1 query: 134 us, 5.7 TB/s).  knn_dist_split_kernel: the flat search's fp32 products of
+// 33 queries on, as bf16 parts (250000 x 768 by 256 queries, us: 778 as fp32, 550 so, of 590 GFLOP of
+// bf16 at the 1.7 GHz this load runs at; by 40: 262 with the selection, now 217; 30000 x 768 by 256: 123, 100).
+// knn_dist_small_kernel: 32 rows x 32 queries a workgroup with K split over
 // its 4 or 8 waves, operands straight from memory: the shapes whose 128-row tiles leave CUs idle
 // are bound by the latency of one K walk, which this cuts (dist_plan).
 #pragma once
@@ -32,6 +35,7 @@ struct DistArgs {
   float* D;
   float* mins;           // TILED: [nq, ldt]
   int n, nq, rowbytes, ldt, mode;
+  const void* parts;     // the queries for knn_dist_split_kernel (knn_split_kernel's)
 };
 
 // 16-B chunk `ch` of `row` in a [rows][128 B] tile: 32-row fragment reads hit distinct banks
@@ -100,6 +104,212 @@ __device__ __forceinline__ float dist_put(const DistArgs& p, int row, int q, con
 }
 
 constexpr int kDistRows = 128;
+
+// ---- fp32 as three bf16 parts.  Every value is the exact sum of three bf16 ones (8 + 8 + 8 bits, each rounded
+// to nearest); of the nine products of two values the six down to 2^-16 of the largest run on the bf16 matrix
+// cores, 16 times as fast as fp32's.  What is left out is 2^-25 of a product, and the sum has fewer roundings
+// than an fp32 one (K / 16 x 6 for K / 2).  Against 64 bits, rms of the 10 nearest's distances, fp32 products /
+// these: 100000 unit rows of 384 1.26e-7 / 1.11e-7, of 768 1.34e-7 / 1.16e-7, inner products 6.1e-8 / 5.1e-8.
+__device__ __forceinline__ void dist_split(const uint4 (&x)[2], bf16x8 (&s)[3]) {
+  uint32_t p[3][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint4& v = x[i >> 1];
+    float a = __uint_as_float(i & 1 ? v.z : v.x), b = __uint_as_float(i & 1 ? v.w : v.y);
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      p[t][i] = pack2(a, b);
+      a -= __uint_as_float(p[t][i] << 16);
+      b -= __uint_as_float(p[t][i] & 0xffff0000u);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < 3; ++t) s[t] = __builtin_bit_cast(bf16x8, make_uint4(p[t][0], p[t][1], p[t][2], p[t][3]));
+}
+
+// A query's parts: 12 pieces of 16 bytes for 32 values (zeros past the end), piece (2 * 3 w + part 2 + h) the 8 values
+// 16 w + 4 h .. + 3 and 16 w + 8 + 4 h .. + 3: what a fragment's lane half h holds of the database's fp32
+inline int dist_parts_bytes(int rowbytes) { return (rowbytes + 127) / 128 * 192; }
+
+static __global__ __launch_bounds__(256) void knn_split_kernel(const float* __restrict__ x, char* __restrict__ y, int nq, int d,
+                                                        int blocks) {
+  const long long e = (long long)blockIdx.x * 256 + threadIdx.x;
+  const long long q = e / (blocks * 4);
+  const int u = (int)(e % (blocks * 4)), w = u >> 1, h = u & 1;   // 16 values' half
+  if (q >= nq) return;
+  uint4 v[2];
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    const int k = w * 16 + g * 8 + h * 4;                         // d % 8 == 0: wholly inside or wholly past
+    v[g] = k < d ? *reinterpret_cast<const uint4*>(x + q * d + k) : make_uint4(0, 0, 0, 0);
+  }
+  bf16x8 s[3];
+  dist_split(v, s);
+  char* o = y + q * (blocks * 192) + (w >> 1) * 192 + (w & 1) * 96 + h * 16;
+#pragma unroll
+  for (int t = 0; t < 3; ++t) *reinterpret_cast<bf16x8*>(o + t * 32) = s[t];
+}
+
+// 128 rows x QT queries a workgroup, a wave 32 rows: rows arrive as fp32 and are split once, by the wave that
+// owns them (44 instructions for QT / 32 x 6 MFMAs of 32 clocks), the queries' parts as they are.  (Waves of
+// 64 x 64, each row split by two: 657 us for 612 with the selection; 8 waves on 256 rows 626.)
+template <int QT>
+__global__ __launch_bounds__(256, 2) void knn_dist_split_kernel(DistArgs p, int nqt) {
+  constexpr int QI = QT / 32, LA = kDistRows / 32, LQ = QT * 12 / 256;   // 16-B loads a thread and stage
+  constexpr int SA = kDistRows * 128, STAGE = SA + QT * 192, NS = 2;   // 80 / 56 KB
+  static_assert(NS * STAGE <= 80 * 1024, "two workgroups a CU");
+  __shared__ __attribute__((aligned(16))) char smem[NS * STAGE];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hh = lane >> 5;
+  const int wg = xcd_remap(blockIdx.x, gridDim.x);      // a row tile's query tiles share an XCD's L2
+  const int row0 = (wg / nqt) * kDistRows, q0 = (wg % nqt) * QT;
+  const int nch = p.rowbytes >> 4, nk = (nch + 7) >> 3, qbytes = nk * 192;
+  const uint32_t lds = lds_u32(smem);
+
+  const char* xt = (const char*)p.xb + (size_t)row0 * p.rowbytes;
+  const char* qt = (const char*)p.parts + (size_t)q0 * qbytes;
+  uint32_t off[LA], offq[LQ];
+  const int lch = (tid & 7) ^ ((tid >> 4) & 7);
+#pragma unroll
+  for (int i = 0; i < LA; ++i)
+    off[i] = (uint32_t)(min(i * 32 + (tid >> 3), p.n - 1 - row0) * p.rowbytes + lch * 16);
+#pragma unroll
+  for (int i = 0; i < LQ; ++i) {
+    const int c = i * 256 + tid, r = c / 12;            // piece x of row r lies at x ^ (r >> 2 & 3): 16 rows' pieces
+    offq[i] = (uint32_t)(min(r, p.nq - 1 - q0) * qbytes + ((c % 12) ^ ((r >> 2) & 3)) * 16);   // hit distinct banks
+  }
+  auto stage = [&](int kt, int buf) {
+    const uint32_t base = lds + (uint32_t)(buf * STAGE + wave * 1024);
+    // chunks past the row's end: its first ones, valid memory that no product reads
+    const uint32_t at = kt * 8 + lch < nch ? (uint32_t)kt * 128 : 0u - (uint32_t)lch * 16;
+#pragma unroll
+    for (int i = 0; i < LA; ++i) glds16_off(xt, off[i] + at, __builtin_amdgcn_readfirstlane(base + (uint32_t)(i * 4096)));
+#pragma unroll
+    for (int i = 0; i < LQ; ++i)
+      glds16_off(qt, offq[i] + (uint32_t)kt * 192, __builtin_amdgcn_readfirstlane(base + (uint32_t)(SA + i * 4096)));
+  };
+  const float f0 = tid < kDistRows ? dist_first(p, row0 + tid) : 0.f;   // (before the ring: its waits count loads)
+  f32x16 acc[QI];
+#pragma unroll
+  for (int j = 0; j < QI; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[j][r] = 0.f;
+
+#pragma unroll
+  for (int t = 0; t < NS - 1; ++t)
+    if (t < nk) stage(t, t);
+  int buf = 0, kt = 0;
+  auto arrive = [&]() {
+    if (NS > 2 && kt + 1 < nk) wait_vmcnt<(NS - 2) * (LA + LQ)>();
+    else wait_vmcnt<0>();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    ring_barrier();
+    if (kt + NS - 1 < nk) stage(kt + NS - 1, buf ? buf - 1 : NS - 1);
+  };
+  // 16 values of the wave's rows (8 where not whole, the others 0), and of the queries
+  auto read_a = [&](int w, bool whole, uint4 (&v)[2]) {
+    const char* sa = smem + buf * STAGE;
+#pragma unroll
+    for (int g = 0; g < 2; ++g) v[g] = *reinterpret_cast<const uint4*>(sa + dist_swz(wave * 32 + l32, w * 4 + g * 2 + hh));
+    if (!whole) v[1] = make_uint4(0, 0, 0, 0);
+  };
+  auto read_b = [&](int w, bf16x8 (&b)[QI][3]) {
+    const char* sq = smem + buf * STAGE + SA;
+#pragma unroll
+    for (int j = 0; j < QI; ++j)
+#pragma unroll
+      for (int t = 0; t < 3; ++t)
+        b[j][t] = *reinterpret_cast<const bf16x8*>(sq + (j * 32 + l32) * 192 +
+                                                   (((w * 3 + t) * 2 + hh) ^ ((l32 >> 2) & 3)) * 16);
+  };
+  auto mma = [&](const bf16x8 (&a)[3], const bf16x8 (&b)[QI][3]) {
+    constexpr int TA[6] = {2, 0, 1, 1, 0, 0}, TB[6] = {0, 2, 1, 0, 1, 0};   // the small products first
+#pragma unroll
+    for (int t = 0; t < 6; ++t)
+#pragma unroll
+      for (int j = 0; j < QI; ++j)
+        acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[TA[t]], b[j][TB[t]], acc[j], 0, 0, 0);
+  };
+  // whole steps in a loop of their own, as above; the second half's parts are made between the first's products
+  for (; kt < nch >> 3; ++kt) {
+    arrive();
+    uint4 v0[2], v1[2];
+    bf16x8 a0[3], a1[3], b0[QI][3], b1[QI][3];
+    read_a(0, true, v0);
+    read_b(0, b0);
+    read_a(1, true, v1);
+    dist_split(v0, a0);
+    __builtin_amdgcn_sched_barrier(0);
+    mma(a0, b0);
+    read_b(1, b1);
+    dist_split(v1, a1);
+#pragma unroll
+    for (int i = 0; i < 3 * QI; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);          // a product
+      __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);          // two vector instructions
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);          // an LDS read
+      __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    mma(a1, b1);
+    buf = buf + 1 == NS ? 0 : buf + 1;
+  }
+  if (kt < nk) {
+    arrive();
+    const int left = (nch - kt * 8) >> 1;               // 8 values each
+    for (int u = 0; u < left; u += 2) {
+      uint4 v[2];
+      bf16x8 a[3], b[QI][3];
+      read_a(u >> 1, u + 1 < left, v);
+      read_b(u >> 1, b);
+      dist_split(v, a);
+      mma(a, b);
+    }
+  }
+
+  // values that came out infinite or NaN (the parts of such an operand, or a large one's products, do) are
+  // what fp32 products make them, straight from memory
+#pragma unroll
+  for (int j = 0; j < QI; ++j) {
+    bool bad = false;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) bad = bad || !(fabsf(acc[j][r]) < INFINITY);
+    if (!__any(bad)) continue;
+    f32x16 e[1][1];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) e[0][0][r] = 0.f;
+    const char* ar = xt + (size_t)min(wave * 32 + l32, p.n - 1 - row0) * p.rowbytes + hh * 16;
+    const char* br = (const char*)p.xq + (size_t)min(q0 + j * 32 + l32, p.nq - 1) * p.rowbytes + hh * 16;
+    for (int g = 0; g < p.rowbytes; g += 32) {
+      const uint4 a[1] = {*reinterpret_cast<const uint4*>(ar + g)}, b[1] = {*reinterpret_cast<const uint4*>(br + g)};
+      dist_mma<false, 1, 1>(a, b, e);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      if (!(fabsf(acc[j][r]) < INFINITY)) acc[j][r] = e[0][0][r];
+  }
+
+  __syncthreads();                                      // the ring is free: the rows' first terms
+  float* first = reinterpret_cast<float*>(smem);
+  if (tid < kDistRows) first[tid] = f0;
+  __syncthreads();
+  const float c = dist_factor(p);
+  const int lt = wave * 32, tile = row0 + lt;
+#pragma unroll
+  for (int j = 0; j < QI; ++j) {
+    const int q = q0 + j * 32 + l32;
+    float mn = FLT_MAX;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float4 f = *reinterpret_cast<const float4*>(first + lt + 8 * g + 4 * hh);
+      mn = fminf(mn, dist_put<true>(p, tile + 8 * g + 4 * hh, q, f, c, acc[j][4 * g], acc[j][4 * g + 1],
+                                    acc[j][4 * g + 2], acc[j][4 * g + 3]));
+    }
+    mn = fminf(mn, __shfl_xor(mn, 32, 64));
+    if (hh == 0 && q < p.nq && tile < p.n) p.mins[(size_t)q * p.ldt + (tile >> 5)] = mn;
+  }
+}
 
 template <int QT, bool BF16, bool TILED>
 __global__ __launch_bounds__(256, 2) void knn_dist_kernel(DistArgs p, int nqt) {
@@ -277,8 +487,15 @@ inline void dist_launch(const DistArgs& p, hipStream_t s) {
   const int qt = dist_plan(p.n, p.nq, p.rowbytes);
   const int rt = (p.n + kDistRows - 1) / kDistRows;
   auto nt = [&](int w) { return (p.nq + w - 1) / w; };
-  if (qt == 128) knn_dist_kernel<128, BF16, TILED><<<rt * nt(128), 256, 0, s>>>(p, nt(128));
-  else if (qt == 64) knn_dist_kernel<64, BF16, TILED><<<rt * nt(64), 256, 0, s>>>(p, nt(64));
+  if (qt >= 64) {
+    if constexpr (TILED && !BF16) {
+      if (qt == 128) knn_dist_split_kernel<128><<<rt * nt(128), 256, 0, s>>>(p, nt(128));
+      else knn_dist_split_kernel<64><<<rt * nt(64), 256, 0, s>>>(p, nt(64));
+    } else {
+      if (qt == 128) knn_dist_kernel<128, BF16, TILED><<<rt * nt(128), 256, 0, s>>>(p, nt(128));
+      else knn_dist_kernel<64, BF16, TILED><<<rt * nt(64), 256, 0, s>>>(p, nt(64));
+    }
+  }
   else if (qt == 32) knn_dist_kernel<32, BF16, TILED><<<rt * nt(32), 256, 0, s>>>(p, nt(32));
   // 4 waves while each has its share of a row in flight at once, else 8 (fp32, 2647 rows by 32
   // queries, 4 / 8 waves: d 384 6.5 / 8.5 us, d 768 10.3 / 9.1)

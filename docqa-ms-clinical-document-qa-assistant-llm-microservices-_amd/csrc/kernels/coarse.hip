@@ -116,7 +116,7 @@ int docqa_fp32_gemm_nt(const float* x, int nq, int d, const float* w, int n, flo
   if (nq == 0) return 0;
   if (d % 8 != 0 || n <= 0 || !docqa_aligned16(x) || !docqa_aligned16(w)) return -1;
   if ((size_t)32 * d * 4 > 160 * 1024) return -2;        // the widest rows this entry point takes
-  dist_launch<false, false>(DistArgs{w, x, nullptr, out, nullptr, n, nq, d * 4, 0, DIST_DOT}, s);
+  dist_launch<false, false>(DistArgs{w, x, nullptr, out, nullptr, n, nq, d * 4, 0, DIST_DOT, nullptr}, s);
   DOCQA_CHECK_LAUNCH();
   return 0;
 }
@@ -129,7 +129,7 @@ int docqa_coarse_probes(const float* cent, const float* cnorm, int nlist, int d,
   if (d % 8 != 0 || nlist <= 0 || nprobe < 1 || nprobe > kMaxProbe || nprobe > nlist) return -1;
   if (!docqa_aligned16(cent) || !docqa_aligned16(xq)) return -1;
   if ((size_t)32 * d * 4 > 160 * 1024) return -2;
-  dist_launch<false, false>(DistArgs{cent, xq, cnorm, ws, nullptr, nlist, nq, d * 4, 0, DIST_L2}, s);
+  dist_launch<false, false>(DistArgs{cent, xq, cnorm, ws, nullptr, nlist, nq, d * 4, 0, DIST_L2, nullptr}, s);
   coarse_select_kernel<<<nq, 256, 0, s>>>(ws, nlist, nprobe, probes);
   DOCQA_CHECK_LAUNCH();
   return 0;

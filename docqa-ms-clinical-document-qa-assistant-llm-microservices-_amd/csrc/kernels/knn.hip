@@ -158,8 +158,11 @@ __global__ __launch_bounds__(256) void knn_round_kernel(const float* __restrict_
 constexpr long long kPiece = 64ll << 20;     // distances a launch may leave in the workspace: 268 MB
 }  // namespace
 
+// pieces of n rows and c queries run on the queries' bf16 parts
+static bool knn_splits(int n, int c, int d, int is_bf16) { return !is_bf16 && dist_plan(n, c, d * 4) >= 64; }
+
 // queries and rows of a piece, and the workspace in bytes (docqa_knn lays it out):
-// distances, minima, carried keys, rounded queries
+// distances, minima, carried keys, rounded queries or the parts of a piece's
 void docqa_knn_plan(int N, int nq, int d, int is_bf16, int k, int* qc, int* rc, size_t* bytes) {
   const long long n32 = ((long long)N + 31) / 32 * 32;
   long long c = nq, r = n32;
@@ -171,6 +174,7 @@ void docqa_knn_plan(int N, int nq, int d, int is_bf16, int k, int* qc, int* rc, 
   *qc = (int)c;
   *rc = (int)r;
   *bytes = (size_t)c * r * 4 + (size_t)c * (r / 32) * 4 + 16 + (size_t)c * k * 8 + (is_bf16 ? (size_t)nq * d * 2 : 0);
+  if (knn_splits(*rc < N ? *rc : N, *qc, d, is_bf16)) *bytes += (size_t)*qc * dist_parts_bytes(d * 4) + 16;
 }
 
 // xb / xq 16-byte aligned; k <= 64
@@ -196,14 +200,22 @@ int docqa_knn(const void* xb, const float* norms, int N, int d, int is_bf16, con
   u64* carry = (u64*)at;
   at += (size_t)qc * k * 8;
   float* mins = (float*)at;
+  at += (size_t)qc * (rc / 32) * 4;
+  void* parts = nullptr;
+  if (knn_splits(rc < N ? rc : N, qc, d, is_bf16)) parts = (void*)(((uintptr_t)at + 15) & ~(uintptr_t)15);
   for (int q0 = 0; q0 < nq; q0 += qc) {
     const int c = nq - q0 < qc ? nq - q0 : qc;
     const float* xs = xq + (size_t)q0 * d;
+    if (parts) {
+      const int blocks = (d + 31) / 32;
+      knn_split_kernel<<<(unsigned)(((long long)c * blocks * 4 + 255) / 256), 256, 0, s>>>(xs, (char*)parts, c, d, blocks);
+    }
     for (int r0 = 0; r0 < N; r0 += rc) {
       const int n = N - r0 < rc ? N - r0 : rc, T = (n + 31) / 32;
       DistArgs p{(const char*)xb + (size_t)r0 * rowbytes,
                  is_bf16 ? (const void*)((const uint16_t*)q16 + (size_t)q0 * d) : (const void*)xs,
-                 metric_ip ? nullptr : norms + r0, D, mins, n, c, rowbytes, T, metric_ip ? DIST_IP : DIST_L2};
+                 metric_ip ? nullptr : norms + r0, D, mins, n, c, rowbytes, T, metric_ip ? DIST_IP : DIST_L2,
+                 parts};
       if (is_bf16) dist_launch<true, true>(p, s);
       else dist_launch<false, true>(p, s);
       knn_select_kernel<<<c, 256, 0, s>>>(D, mins, T, T, c, k, (uint32_t)r0, carry, r0 == 0, n == N - r0, xs, d,

@@ -29,6 +29,7 @@ def _check(xb, xq, k, ip, offset=0):
 @pytest.mark.parametrize("N,nq,d", [
     (1, 1, 8), (31, 3, 24), (32, 33, 40), (33, 1, 384), (2647, 1, 384), (2647, 256, 384),      # small workgroups
     (32641, 1, 104), (40000, 31, 72), (32700, 33, 40), (17000, 65, 48), (33000, 129, 56),      # each tile width
+    (66000, 40, 72), (65537, 64, 40), (70000, 33, 32), (33000, 200, 8),                        # and its row ends
 ])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("k,ip", [(1, False), (10, True), (64, False)])
@@ -119,3 +120,29 @@ def test_refine_widths(d, dtype, metric):
 def test_row_norms():
     x = torch.randn(1001, 37, device="cuda")
     assert torch.allclose(ops.row_norms(x), (x ** 2).sum(1), rtol=1e-5)
+
+
+@pytest.mark.parametrize("ip", [False, True])
+@pytest.mark.parametrize("nq,N", [(150, 33000), (50, 66000)])
+def test_knn_values_at_the_ends(nq, N, ip):
+    """Wide batches multiply fp32 as bf16 parts: rows and queries of infinities, NaN, values beyond bf16's largest,
+    products beyond fp32's and tiny ones come out as the narrow batches' fp32 products make them."""
+    g = torch.Generator(device="cuda").manual_seed(nq)
+    d = 40
+    xb, xq = torch.randn(N, d, device="cuda", generator=g), torch.randn(nq, d, device="cuda", generator=g)
+    inf, big = float("inf"), 3.4e38
+    xb[5, 3], xb[40, 7], xb[41], xb[100, 0], xb[N - 1, 39] = inf, -inf, float("nan"), big, inf
+    xb[200], xb[300, :20], xb[300, 20:] = 1e30, 1e30, -1e30
+    xb[400] *= 1e-30
+    xq[1, 3], xq[2], xq[3, 0], xq[4], xq[nq - 1, 5] = -inf, 1e20, big, 1e-30, float("nan")
+    norms = (xb ** 2).sum(1)
+    D, I = ops.knn(xb, norms, xq, 20, ip, 0)
+    parts = [ops.knn(xb, norms, xq[i:i + 25], 20, ip, 0) for i in range(0, nq, 25)]
+    Dn, In = torch.cat([p[0] for p in parts]), torch.cat([p[1] for p in parts])
+    assert torch.equal(D.isfinite(), Dn.isfinite()) and torch.equal(I < 0, In < 0)
+    assert torch.equal(D[~D.isfinite()].nan_to_num(1.0), Dn[~Dn.isfinite()].nan_to_num(1.0))
+    # 40 products and the norms, each rounded by 2^-24 on either side
+    size = (xq.double() ** 2).sum(1, keepdim=True).nan_to_num(0, 0, 0) + 2000 + Dn.double().abs().nan_to_num(0, 0, 0)
+    assert bool(((D.double() - Dn.double()).abs().nan_to_num(0, 0, 0) <= 40 * 2.0 ** -22 * size).all())
+    ordinary = torch.arange(5, nq - 1, device="cuda")
+    assert torch.equal((I == 400)[ordinary], (In == 400)[ordinary])
