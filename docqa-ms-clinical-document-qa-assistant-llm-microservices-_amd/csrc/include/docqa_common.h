@@ -93,15 +93,29 @@ __device__ __forceinline__ float act_f(float v) {
   return ACT == ACT_RELU2 ? relu2(v) : gelu_tanh(v);
 }
 
+// op over a wave's lanes, in all of them: partners 32, 16, 8, 4, 2, 1 lanes apart (what __shfl_xor would pair, so
+// the same sums), by row swaps and DPP in the vector unit: six round trips through LDS were about 0.3 us of a
+// kernel's chain
+template <int CTRL, int BANKS = 0xf>
+__device__ __forceinline__ float dpp_of(float old, float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), CTRL, 0xf, BANKS, false));
+}
+template <typename F>
+__device__ __forceinline__ float wave_reduce(float v, F op) {
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = op(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = op(__uint_as_float(b[0]), __uint_as_float(b[1]));
+  v = op(v, dpp_of<0x128>(v, v));                                   // row_ror 8
+  v = op(v, dpp_of<0x114, 0xa>(dpp_of<0x104, 0x5>(v, v), v));       // row_shl 4 into banks 0, 2; row_shr 4 into 1, 3
+  v = op(v, dpp_of<0x4e>(v, v));                                    // quad_perm 2 3 0 1
+  return op(v, dpp_of<0xb1>(v, v));                                 // quad_perm 1 0 3 2
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  return wave_reduce(v, [](float x, float y) { return x + y; });
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
+  return wave_reduce(v, [](float x, float y) { return fmaxf(x, y); });
 }
 // value of the lane `N` positions up inside its 16-lane DPP row (row_ror:N), no LDS trip
 template <int N>
