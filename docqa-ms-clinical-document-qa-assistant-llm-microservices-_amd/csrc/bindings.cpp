@@ -282,9 +282,32 @@ at::Tensor bert_hidden(const at::Tensor& ids, const c10::optional<at::Tensor>& p
   CHECK_RC(docqa_bert_embed_ln(ids.data_ptr<int>(), pp, cu, B, nullptr, wte.data_ptr(), wpe.data_ptr(),
                                wtt.data_ptr(), gamma.data_ptr(), beta.data_ptr(), h, M, h_, (float)eps, s),
            "bert_embed_ln");
+  // few rows: a layer's two normalisations run inside the products behind them
+  auto aligned = [](const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) == 0; };
+  bool ln_in = docqa_gemm_ln_ok(M, 3 * h_, h_);
+  for (size_t l = 0; l < layers.size() && ln_in; l += 12) {
+    ln_in = docqa_gemm_ln_ok(M, (int)layers[l + 6].size(0), h_);
+    for (int i = 0; i < 12; ++i) ln_in = ln_in && aligned(layers[l + i]);
+  }
   for (size_t l = 0; l < layers.size(); l += 12) {
     const int I = (int)layers[l + 6].size(0);
     auto p = [&](int i) { return layers[l + i].data_ptr(); };
+    if (ln_in) {
+      if (l == 0) {
+        CHECK_RC(docqa_gemm(h, p(0), p(1), nullptr, qkv, M, 3 * h_, h_, 1, s), "gemm");
+      } else {
+        CHECK_RC(docqa_gemm_ln(sum, layers[l - 2].data_ptr(), layers[l - 1].data_ptr(), (float)eps, h, p(0), p(1), qkv, M,
+                               3 * h_, h_, 1, s), "gemm_ln");
+      }
+      CHECK_RC(docqa_flash_prefill(qkv, 3 * h_, cu, att, h_, B, (int)max_len, (int)heads, (int)heads, D, (float)scale,
+                                   0, s), "flash_prefill");
+      CHECK_RC(docqa_gemm(att, p(2), p(3), h, sum, M, h_, h_, 3, s), "gemm");
+      CHECK_RC(docqa_gemm_ln(sum, p(4), p(5), (float)eps, h, p(6), p(7), up, M, I, h_, 2, s), "gemm_ln");
+      CHECK_RC(docqa_gemm(up, p(8), p(9), h, sum, M, h_, I, 3, s), "gemm");
+      if (l + 12 == layers.size())
+        CHECK_RC(docqa_layernorm(sum, nullptr, p(10), p(11), h, M, h_, (float)eps, s), "layernorm");
+      continue;
+    }
     CHECK_RC(docqa_gemm(h, p(0), p(1), nullptr, qkv, M, 3 * h_, h_, 1, s), "gemm");
     CHECK_RC(docqa_flash_prefill(qkv, 3 * h_, cu, att, h_, B, (int)max_len, (int)heads, (int)heads, D, (float)scale,
                                  0, s), "flash_prefill");

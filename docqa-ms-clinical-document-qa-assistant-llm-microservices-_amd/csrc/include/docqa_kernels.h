@@ -149,6 +149,9 @@ int docqa_dgemm(const void* X, const void* W, void* Y, float* partial, int M, in
                 hipStream_t s);
 int docqa_gemm(const void* A, const void* W, const void* bias, const void* res, void* C, int M,
                int N, int K, int epi, hipStream_t s);
+bool docqa_gemm_ln_ok(int M, int N, int K);
+int docqa_gemm_ln(const void* X, const void* gamma, const void* beta, float eps, void* A, const void* W, const void* bias,
+                  void* C, int M, int N, int K, int epi, hipStream_t s);
 int docqa_mgemm(const void* X, const void* W, void* Y, float* P, int M, int N, int K, int S, int cfg,
                 hipStream_t s);
 int docqa_mgemm_slab16(const void* X, const void* W, void* Y, int M, int N, int K, int S, int cfg,

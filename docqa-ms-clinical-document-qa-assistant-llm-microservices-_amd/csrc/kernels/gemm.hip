@@ -470,7 +470,189 @@ __global__ __launch_bounds__(256, 2) void gemm_few_kernel(const uint16_t* __rest
     *reinterpret_cast<uint4*>(C + at) = pack8(v);
   }
 }
+// ---- few rows of an encoder layer behind their LayerNorm: A = LN(X) gamma + beta (layernorm_kernel's arithmetic,
+// bit for bit), made by every workgroup for its own 32 rows while its first weights are on the way, so that no
+// launch stands between two products; the first column tile's workgroups also write A, the next residual.  32 x 32
+// tiles, 8 waves normalise, 4 of them multiply with K split as above, A whole in LDS, W in 128-deep stages.  Bound
+// by its chain of latencies; 24 rows of MiniLM, us: up 2.75 + 3.85 -> 6.35, QKV 2.75 + 3.6 -> 5.9, and the gap
+// between two launches less (with 4 waves 6.7 and 6.3).
+constexpr int LN_MAXK = 768;    // 80 KB of LDS, two workgroups a CU
+template <int EPI, int NV>
+__global__ __launch_bounds__(512) void gemm_few_ln_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ gamma,
+                                                          const uint16_t* __restrict__ beta, float eps,
+                                                          uint16_t* __restrict__ A, const uint16_t* __restrict__ W,
+                                                          const uint16_t* __restrict__ bias, uint16_t* __restrict__ C, int M,
+                                                          int N, int K) {
+  constexpr int T = 32, STAGE = T * 256, NS = 4, PITCH = T + 4;
+  constexpr int PANEL = T * (NV == 1 ? 512 : LN_MAXK) * 2;
+  __shared__ __attribute__((aligned(16))) char smem[PANEL + NS * STAGE];
+  static_assert(4 * T * PITCH * 4 <= PANEL + NS * STAGE, "partial sums");
+  const int nbn = N / T;
+  const int wg = xcd_remap(blockIdx.x, gridDim.x);
+  const int row0 = (wg / nbn) * T, col0 = (wg % nbn) * T;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hh = lane >> 5;
+  char* ring = smem + PANEL;
+  const uint32_t lds = lds_u32(ring);
+  const char* wb = (const char*)(W + (size_t)col0 * K);
+  const uint32_t off = (uint32_t)(tid >> 4) * (uint32_t)(K * 2) + (uint32_t)((tid & 15) ^ ((tid >> 4) & 15)) * 16;
+  auto stage = [&](int kt, int buf) {                // 16 bytes a thread
+    glds16_off(wb, off + (uint32_t)kt * 256, __builtin_amdgcn_readfirstlane(lds + (uint32_t)(buf * STAGE + wave * 1024)));
+  };
+  const int nk = K / 128, nchunk = K >> 3;
+#pragma unroll
+  for (int t = 0; t < NS - 1; ++t)
+    if (t < nk) stage(t, t);
+
+  // a wave normalises 4 rows (rows past the end: the last one again, never stored)
+  uint4 raw[4][NV], gr[NV], br[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = min(lane + 64 * i, nchunk - 1);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      raw[r][i] = reinterpret_cast<const uint4*>(X + (size_t)min(row0 + wave * 4 + r, M - 1) * K)[c];
+    gr[i] = reinterpret_cast<const uint4*>(gamma)[c];
+    br[i] = reinterpret_cast<const uint4*>(beta)[c];
+  }
+  float mean[4], inv[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      float v[8];
+      unpack8(raw[r][i], v);
+      if (lane + 64 * i < nchunk) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s += v[j];
+      }
+    }
+    mean[r] = s;
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) mean[r] = wave_sum(mean[r]) / (float)K;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      float v[8];
+      unpack8(raw[r][i], v);
+      if (lane + 64 * i < nchunk) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float d = v[j] - mean[r];
+          ss += d * d;
+        }
+      }
+    }
+    inv[r] = ss;
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) inv[r] = rsqrtf(wave_sum(inv[r]) / (float)K + eps);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = lane + 64 * i;
+    if (c >= nchunk) continue;
+    float g[8], b[8];
+    unpack8(gr[i], g);
+    unpack8(br[i], b);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = wave * 4 + r;
+      float v[8], o[8];
+      unpack8(raw[r][i], v);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o[j] = (v[j] - mean[r]) * inv[r] * g[j] + b[j];
+      const uint4 p = pack8(o);
+      *reinterpret_cast<uint4*>(smem + row * (K * 2) + (((c & ~15) | ((c & 15) ^ (row & 15))) << 4)) = p;
+      if (col0 == 0 && row0 + row < M) reinterpret_cast<uint4*>(A + (size_t)(row0 + row) * K)[c] = p;
+    }
+  }
+
+  f32x16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  int buf = 0;
+  for (int kt = 0; kt < nk; ++kt) {
+    // (the rows' stores, issued after the first stages, only make these waits longer)
+    const int later = min(NS - 2, nk - 1 - kt);
+    if (later == 2) wait_vmcnt<2>();
+    else if (later == 1) wait_vmcnt<1>();
+    else wait_vmcnt<0>();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    ring_barrier();
+    if (kt + NS - 1 < nk) stage(kt + NS - 1, buf ? buf - 1 : NS - 1);
+    if (wave < 4) {
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        const int ch = ((wave * 2 + ks) * 2 + hh) ^ (l32 & 15);
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(smem + l32 * (K * 2) + kt * 256 + ch * 16);
+        const bf16x8 w = *reinterpret_cast<const bf16x8*>(ring + buf * STAGE + l32 * 256 + ch * 16);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, a, acc, 0, 0, 0);
+      }
+    }
+    buf = buf == NS - 1 ? 0 : buf + 1;
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  ring_barrier();                                    // the partial sums' place now
+  float* part = reinterpret_cast<float*>(smem);
+  if (wave < 4) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<f32x4*>(part + (wave * T + l32) * PITCH + 8 * g + 4 * hh) =
+          f32x4{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+  }
+  __syncthreads();
+  const int r = tid >> 2, c = (tid & 3) * 8;
+  if (r >= T || row0 + r >= M) return;
+  float v[8] = {};
+#pragma unroll
+  for (int w = 0; w < 4; ++w)
+#pragma unroll
+    for (int e = 0; e < 8; e += 4) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(part + (w * T + r) * PITCH + c + e);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[e + k] += x[k];
+    }
+  float b[8];
+  unpack8(*reinterpret_cast<const uint4*>(bias + col0 + c), b);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    v[e] += b[e];
+    if constexpr (EPI == EPI_BIAS_GELU) v[e] = gelu_erf(v[e]);
+  }
+  *reinterpret_cast<uint4*>(C + (size_t)(row0 + r) * N + col0 + c) = pack8(v);
+}
 }  // namespace
+
+// whether docqa_gemm_ln takes the product: as few 32 x 32 tiles as docqa_gemm gives that form
+bool docqa_gemm_ln_ok(int M, int N, int K) {
+  return M > 0 && N % BN == 0 && K % 128 == 0 && K <= LN_MAXK && (long long)((M + 31) / 32) * (N / 32) <= 512;
+}
+
+// C = act(A . W^T + bias), A = LN(X) gamma + beta, which is written too; epi bias or bias + GELU.  X and A differ.
+int docqa_gemm_ln(const void* X, const void* gamma, const void* beta, float eps, void* A, const void* W, const void* bias,
+                  void* C, int M, int N, int K, int epi, hipStream_t s) {
+  if (!docqa_gemm_ln_ok(M, N, K) || (epi != EPI_BIAS && epi != EPI_BIAS_GELU) || X == A) return -1;
+  for (const void* p : {X, gamma, beta, (const void*)A, W, bias, (const void*)C})
+    if (!docqa_aligned16(p)) return -1;
+  const int grid = (M + 31) / 32 * (N / 32);
+#define DOCQA_LN(E, NV)                                                                                                   \
+  gemm_few_ln_kernel<E, NV><<<grid, 512, 0, s>>>((const uint16_t*)X, (const uint16_t*)gamma, (const uint16_t*)beta, eps, \
+                                                 (uint16_t*)A, (const uint16_t*)W, (const uint16_t*)bias, (uint16_t*)C, M, N, K)
+  if (K <= 512) {
+    if (epi == EPI_BIAS) DOCQA_LN(EPI_BIAS, 1);
+    else DOCQA_LN(EPI_BIAS_GELU, 1);
+  } else {
+    if (epi == EPI_BIAS) DOCQA_LN(EPI_BIAS, 2);
+    else DOCQA_LN(EPI_BIAS_GELU, 2);
+  }
+#undef DOCQA_LN
+  DOCQA_CHECK_LAUNCH();
+  return 0;
+}
 
 // What `tiles` ring tiles take, in eighths of a round of 512 (two workgroups a CU): alone on its CU a workgroup
 // takes five of them.  A round of 192-row tiles is worth 0.8 of one of 256 (fitted to 95 launches, bge-base and

@@ -1,14 +1,14 @@
-"""The encoder stack issued by one call runs the op-by-op path's kernels: its results are the same bytes,
-with positions taken from the sequence starts on the device."""
+"""The encoder stack issued by one call computes what the op-by-op path does, byte for byte: positions taken from
+the sequence starts on the device, and for few rows the normalisations inside the products behind them."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("preset", ["tiny-bert", "minilm-l6"])
-@pytest.mark.parametrize("lengths", [[1], [24], [0, 3, 0, 0, 70, 1, 0], [2] * 63 + [5], [1, 3] * 40, [0, 1, 2] * 1500],
-                         ids=["one", "question", "empty", "64", "80", "4500"])
+@pytest.mark.parametrize("preset", ["tiny-bert", "minilm-l6", "bge-base"])
+@pytest.mark.parametrize("lengths", [[1], [24], [0, 3, 0, 0, 70, 1, 0], [2] * 63 + [5], [1, 3] * 40, [100, 124], [120] * 4, [0, 1, 2] * 1500],
+                         ids=["one", "question", "empty", "64", "80", "224", "480", "4500"])
 def test_stack_equals_its_ops(preset, lengths):
     from docqa_amd import ops
     from docqa_amd.models.bert import BertConfig, BertEncoder, pack, packed_positions
@@ -40,3 +40,19 @@ def test_pack_takes_what_torch_takes():
     assert ids.tolist() == [1, 2, 1, 7, 2, 5] and cu.tolist() == [0, 2, 2, 4, 6] and longest == 2
     assert ids.dtype == cu.dtype == torch.int32
     assert [t.tolist() for t in pack([], 8, "cpu")[:2]] == [[], [0]]
+
+
+@pytest.mark.parametrize("H", [8, 384, 512, 520, 1024])
+def test_pool_lengths(H):
+    from docqa_amd import ops
+
+    lens = [1, 0, 7, 8, 33, 2, 70]
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32, device="cuda")
+    h = torch.randn(sum(lens), H, device="cuda", dtype=torch.bfloat16)
+    for mean in (True, False):
+        got = ops.pool_l2(h, cu, mean, False)
+        for b, n in enumerate(lens):
+            x = h[int(cu[b]):int(cu[b]) + n].double()
+            want = (x.mean(0) if mean else x[0]) if n else torch.zeros(H, device="cuda", dtype=torch.float64)
+            # sums of n bf16 values in fp32, once divided
+            assert bool(((got[b].double() - want).abs() <= (n + 2) * 2.0 ** -24 * (x.abs().mean(0) if n else 0)).all())
