@@ -580,7 +580,8 @@ int launch_mfma(const void* q, const void* kc, const void* vc, void* out, const 
 }
 
 // decode-like launches (the rows of one sequence fit one 16-row tile): waves split the keys, as
-// many to a workgroup as give a CU 16 of them
+// many to a workgroup as give a CU 16 of them; at 128 dimensions 8, for 16 leave a lane 128 registers and
+// spill (32 sequences of 300..1500 tokens, window 1024, 8 KV heads: 16 waves 31.6 us, 8 25.4; 1 sequence 20.3, 19.2)
 template <int DP, int DPV, bool SHARED>
 int dispatch_mfma(const void* q, const void* kc, const void* vc, void* out, const WindowArgs& a, int B, int max_q,
                   hipStream_t s) {
@@ -588,7 +589,7 @@ int dispatch_mfma(const void* q, const void* kc, const void* vc, void* out, cons
   if (max_q * (a.H / a.G) <= 16) {
     if constexpr (DP <= 128 && DPV <= 128) {
       const long long wgs = (long long)B * a.G;
-      if constexpr (SHARED) {
+      if constexpr (SHARED && DP < 128) {
         if (wgs <= 256) return launch_mfma<DP, DPV, 1, 32, 16, SHARED, true>(q, kc, vc, out, a, B, max_q, s);
       }
       if (wgs <= 512) return launch_mfma<DP, DPV, 1, 32, 8, SHARED, true>(q, kc, vc, out, a, B, max_q, s);
