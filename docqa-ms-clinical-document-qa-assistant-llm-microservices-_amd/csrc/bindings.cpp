@@ -235,7 +235,7 @@ at::Tensor bert_embed_ln(const at::Tensor& ids, const at::Tensor& pos,
 // input's kernels (3 - 5 us each) end before the next could be issued op by op.  `layers` holds 12 tensors
 // a layer: qkv w b, o w b, ln1 g b, up w b, down w b, ln2 g b.  One workspace: QKV and the attention's
 // result share their place with the up-projection, which is written after both are read.  One 24-token
-// text through MiniLM's 6 layers: 353 us op by op with positions from torch operators, 171 us so.
+// text through MiniLM's 6 layers: 353 us op by op with positions from torch operators, 171 us so, 152 with the normalisations inside the products.
 at::Tensor bert_hidden(const at::Tensor& ids, const c10::optional<at::Tensor>& pos, const at::Tensor& cu_seqlens,
                        int64_t max_len, const at::Tensor& wte, const at::Tensor& wpe, const at::Tensor& wtt,
                        const at::Tensor& gamma, const at::Tensor& beta, at::TensorList layers, int64_t heads,

@@ -472,8 +472,9 @@ __global__ __launch_bounds__(64 * NW) void knn_dist_small_kernel(DistArgs p, int
 // about one a CU and a K walk is long enough to be worth cutting (us, small / 32-wide: fp32 d 384
 // 8192 rows x 32 queries, 256 workgroups, 6.8 / 10.5, 2647 x 128, 332 of them, 9.5 / 10.2, 16384 x 33,
 // 1024 of them, 18.1 / 10.5; bf16 d 768 2647 x 1 4.2 / 5.8, d 384 2647 x 33 5.2 / 4.3); else the
-// widest tile that still has two workgroups a CU (32 / 64 / 128, fp32 d 384: 16384 x 256 32.8 /
-// 30.8 / 31.1; 32768 x 256 62.1 / 57.3 / 55.1; 8192 x 256 17.8 / 18.0 / 29.0).
+// widest tile that still has two workgroups a CU (32 as fp32 / 64 / 128 as parts, whole searches, fp32 d 384:
+// 8192 x 256 31.6 / 32.2 / 36.9; 16384 x 256 47.7 / 40.6 / 41.2; 32768 x 256 76.8 / 60.0 / 55.1; d 768, 65536 x 48
+// 71 / 59 / 78, x 100 126 / 95 / 84).
 inline int dist_plan(int n, int nq, int rowbytes) {
   const long long rt = (n + kDistRows - 1) / kDistRows;
   if ((long long)((n + 31) / 32) * ((nq + 31) / 32) <= 320 && rowbytes >= 1024) return 0;
